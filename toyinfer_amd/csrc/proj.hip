@@ -15,13 +15,15 @@
 //    call, carry the non-temporal hint (the lm-head's 1.24 GB then streams
 //    at 6.95 TB/s where plain loads reach 6.2).
 //  * gemm_kernel: MFMA-bound (prefill, T > kGemvMaxTokens).  K in 64-wide
-//    slices double-buffered in LDS by buffer-load DMA, v_mfma_f32_32x32x16_bf16
-//    on 32 x 32 blocks.  256 x 256 tiles (8 waves of 128 x 64) when they
-//    alone fill every CU, else 128 x 128 tiles (4 waves of 64 x 64, two
-//    workgroups per CU).  Tiles are ordered in 8 x 8 groups and the groups
-//    are dealt to XCDs in contiguous runs, so the blocks resident on one XCD
-//    share W and x slices in that XCD's L2.  The results leave through LDS
-//    as whole 16-byte chunks of token rows.
+//    slices through a ring of two to four LDS stages by buffer-load DMA,
+//    v_mfma_f32_32x32x16_bf16 on 32 x 32 blocks.  Nine tile sizes from 64 x 64
+//    to 256 x 256, picked by a cost model of tiles, rounds and slices.  Tiles
+//    are ordered in 8 x 8 groups and the groups are dealt to XCDs in
+//    contiguous runs, so the blocks resident on one XCD share W and x slices
+//    in that XCD's L2.  The results leave through LDS as whole 16-byte chunks
+//    of token rows.
+#include <cmath>
+
 #include "common.hpp"
 #include "kernels.hpp"
 
@@ -170,27 +172,63 @@ constexpr int kGmBK = 64;    // K granularity every GEMM configuration handles
 constexpr int kGmGroup = 8;  // tile groups of 8 x 8
 
 // Block tile BM (tokens) x BN (outputs) on a WGM x WGN grid of waves; each
-// wave owns IM x JN blocks of 32 x 32.  K advances in slices of BK (64 or
-// 128): KS k-steps of 16 per slice.
-template <int BM_, int BN_, int WGM_, int WGN_, int MINB_, int BK_ = 64>
+// wave owns IM x JN blocks of 32 x 32.  K advances in slices of kGmBK (KS
+// k-steps of 16) through a ring of ST LDS stages.
+template <int BM_, int BN_, int WGM_, int WGN_, int MINB_, int ST_>
 struct GmCfg {
-    static constexpr int BM = BM_, BN = BN_, WGM = WGM_, WGN = WGN_, MINB = MINB_, BK = BK_;
+    static constexpr int BM = BM_, BN = BN_, WGM = WGM_, WGN = WGN_, MINB = MINB_, ST = ST_;
+    static constexpr int BK = kGmBK;
     static constexpr int WAVES = WGM * WGN, THREADS = 64 * WAVES;
     static constexpr int IM = BM / WGM / 32, JN = BN / WGN / 32;
     static constexpr int KS = BK / 16, CPR = BK / 8, RPB = 64 / CPR;  // chunks per row, rows per DMA
     static constexpr int A_ELEMS = BM * BK, B_ELEMS = BN * BK;
-    static constexpr int A_DMA = BM / RPB / WAVES, B_DMA = BN / RPB / WAVES;  // per wave
-    static_assert(A_DMA * RPB * WAVES == BM && B_DMA * RPB * WAVES == BN, "DMA split");
-    static_assert(BK == 64 || BK == 128, "slice width");
+    static constexpr int A_BLOCKS = BM / RPB;                  // DMA instructions per slice of A
+    static constexpr int BLOCKS = (BM + BN) / RPB;             // and in all
+    static constexpr int DMAS = (BLOCKS + WAVES - 1) / WAVES;  // of them per wave, rounded up
+    static_assert(ST >= 2 && ST <= 4 && (ST - 2) * DMAS < 64, "ring depth");
+    static_assert(32 * IM * WGM == BM && 32 * JN * WGN == BN, "wave grid");
+    static_assert(A_BLOCKS % WAVES == 0, "a wave's j-th DMA is of A or of B for every wave");
 };
-// 64 x 64 tiles serve grids too small to fill the CUs with larger tiles; with
-// few MFMAs per slice they are latency-bound, so they take 128-wide slices.
-using GmMini = GmCfg<64, 64, 2, 2, 4, 128>;  // 4 waves of 32 x 32
-using GmMini64 = GmCfg<64, 64, 2, 2, 4, 64>;
-using GmSmall = GmCfg<128, 128, 2, 2, 2>;  // 4 waves of 64 x 64, 2 workgroups per CU
-using GmMid = GmCfg<128, 192, 2, 2, 2>;    // 4 waves of 64 x 96, 2 workgroups per CU (80 KB LDS each)
-using GmTall = GmCfg<192, 128, 2, 2, 2>;   // 4 waves of 96 x 64, 2 workgroups per CU (80 KB LDS each)
-using GmLarge = GmCfg<256, 256, 2, 4, 1>;  // 8 waves of 128 x 64
+// The configurations, smallest tile first, each with its cost model (us):
+// `fixed` + rounds * (`round` + slices * (`slice` + `load` * u)), rounds =
+// ceil(tiles / CUs), u = the share of the rounds' CU slots that hold a tile.
+// slice is the time of a K slice while the rest of the chip idles (DMA and
+// operand reads for the small tiles, MFMAs for the large), load what a full
+// chip adds (shared caches, and the clock the power limit leaves).  Fitted
+// to 136 measured problems (T 20-4096, the q/k/v, o, gate/up + SwiGLU and
+// down projections of a 1024- and a 4096-wide layer): within 4-6 % rms of
+// every configuration's time, and the configuration it picks is on average
+// 0.3 % and at most 6 % slower than the fastest one.
+struct GmCost {
+    float fixed, round, slice, load;
+};
+struct GmMini : GmCfg<64, 64, 2, 2, 2, 4> {  // 4 waves of 32 x 32, two workgroups per CU
+    static constexpr GmCost COST{2.05f, 0.40f, 0.141f, 0.0425f};
+};
+struct GmSix : GmCfg<96, 64, 3, 2, 1, 4> {  // 6 waves of 32 x 32
+    static constexpr GmCost COST{1.2f, 1.9f, 0.175f, 0.076f};
+};
+struct GmFlat : GmCfg<128, 64, 4, 2, 1, 4> {  // 8 waves of 32 x 32
+    static constexpr GmCost COST{0.8f, 2.1f, 0.174f, 0.114f};
+};
+struct GmDeep : GmCfg<128, 128, 2, 4, 1, 4> {  // 8 waves of 64 x 32
+    static constexpr GmCost COST{0.6f, 3.4f, 0.260f, 0.185f};
+};
+struct GmTall : GmCfg<192, 128, 2, 4, 1, 3> {  // 8 waves of 96 x 32
+    static constexpr GmCost COST{0.0f, 5.9f, 0.322f, 0.279f};
+};
+struct GmHalf : GmCfg<256, 128, 4, 2, 1, 3> {  // 8 waves of 64 x 64
+    static constexpr GmCost COST{0.0f, 7.5f, 0.416f, 0.343f};
+};
+struct GmWide : GmCfg<192, 192, 2, 6, 1, 3> {  // 12 waves of 96 x 32
+    static constexpr GmCost COST{0.0f, 7.6f, 0.428f, 0.431f};
+};
+struct GmBroad : GmCfg<256, 192, 4, 2, 1, 2> {  // 8 waves of 64 x 96
+    static constexpr GmCost COST{0.0f, 7.0f, 0.713f, 0.434f};
+};
+struct GmLarge : GmCfg<256, 256, 2, 4, 1, 2> {  // 8 waves of 128 x 64
+    static constexpr GmCost COST{0.0f, 8.9f, 0.863f, 0.569f};
+};
 
 // LDS rows of BK bf16 (CPR 16-byte chunks); chunk c of row r sits at
 // c ^ gm_swz<CPR>(r).  A 16-byte LDS read serves 16 lanes per cycle from
@@ -206,19 +244,6 @@ using GmLarge = GmCfg<256, 256, 2, 4, 1>;  // 8 waves of 128 x 64
 template <int CPR>
 __device__ __forceinline__ uint32_t gm_swz(uint32_t row) {
     return CPR == 16 ? row & 15 : (row >> 1) & 7;
-}
-
-template <int WAVES, int BLOCKS, int CPR>
-__device__ __forceinline__ void gm_dma(__amdgpu_buffer_rsrc_t r, uint32_t row_bytes, uint32_t k_off,
-                                       uint16_t* lds) {
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-#pragma unroll
-    for (int j = 0; j < BLOCKS; ++j) {
-        const int blk = wave + WAVES * j;
-        const uint32_t row = (64 / CPR) * blk + lane / CPR;
-        const uint32_t logical = (lane % CPR) ^ gm_swz<CPR>(row);
-        dma16(r, lds + 512 * blk, row * row_bytes + k_off + 16 * logical);
-    }
 }
 
 struct GmTile {
@@ -258,11 +283,13 @@ __device__ __host__ __forceinline__ uint32_t gm_out_tiles(const GemmArgs& g) {
 // same banks, the chunk takes bits 1-3 of t and the half bit 0; with 64- or
 // 192-byte rows (CR 4, 12) bit 0 of t picks the 64-byte half of the bank
 // line, the chunk takes bits 1-2 (within its aligned group of four) and the
-// half bit 3.  The 16-byte read-back (16 lanes per cycle from 64 banks) of
-// consecutive chunks of a row stays a permutation of the row's banks.
+// half bit 3; with 32- or 96-byte rows (CR 2, 6) bits 0-1 pick the quarter,
+// the chunk takes bit 2 (within its pair) and the half bit 3.  The 16-byte
+// read-back (16 lanes per cycle from 64 banks) of consecutive chunks of a
+// row stays a permutation of the row's banks.
 template <int CR>
 __device__ __forceinline__ int ep_chunk(int c, int t) {
-    return CR == 8 ? c ^ ((t >> 1) & 7) : c ^ ((t >> 1) & 3);
+    return CR == 8 ? c ^ ((t >> 1) & 7) : (CR % 4 ? c ^ ((t >> 2) & 1) : c ^ ((t >> 1) & 3));
 }
 template <int CR>
 __device__ __forceinline__ int ep_swap(int t) {
@@ -286,7 +313,12 @@ template <int N>
 __device__ __forceinline__ void ep_read(uint4 (&x)[N], const uint32_t (&a)[N]) {
     typedef unsigned v4u_t __attribute__((ext_vector_type(4)));
     v4u_t v[N];
-    if constexpr (N == 2) {
+    if constexpr (N == 1) {
+        asm volatile("ds_read_b128 %0, %1\n\ts_waitcnt lgkmcnt(0)"
+                     : "=&v"(v[0])
+                     : "v"(a[0])
+                     : "memory");
+    } else if constexpr (N == 2) {
         asm volatile("ds_read_b128 %0, %2\n\tds_read_b128 %1, %3\n\ts_waitcnt lgkmcnt(0)"
                      : "=&v"(v[0]), "=&v"(v[1])
                      : "v"(a[0]), "v"(a[1])
@@ -332,20 +364,49 @@ __device__ __forceinline__ uint4 add_bf16x8(uint4 a, uint4 b) {
     return make_uint4(o[0], o[1], o[2], o[3]);
 }
 
-// SW (SwiGLU epilogue): B tile row r belongs to 32-row block b = r / 32;
-// even blocks are gate rows, odd blocks up rows, both of output columns
-// m0 + 32 (b / 2) + r % 32, so a wave's two column blocks (JN = 2) hold
-// gate and up of the same 32 columns and the epilogue pairs them in-lane.
+// DMA instruction `blk` of a slice fills the 64 / CPR tile rows from
+// (64 / CPR) blk on (the A rows, then the B rows) of the stage at st; lane l
+// loads row l / CPR's physical chunk l % CPR, i.e. logical chunk (l % CPR) ^
+// gm_swz<CPR>(row).  SW: 16 gate and 16 up rows make a 32-row block of B,
+// positions p with bit 3 clear gate, the others up, both of the 16 output
+// columns 8 (p / 16) + p % 8, so that a lane's accumulator values 8 q + u
+// and 8 q + 4 + u (u < 4) are gate and up of one output; the eight rows of
+// a DMA instruction are all of one kind.
+template <typename C, bool SW>
+__device__ __forceinline__ uint32_t gm_dma_offset(uint32_t blk, int lane, uint32_t row_bytes) {
+    const uint32_t r = C::RPB * blk + lane / C::CPR;  // tile row
+    const uint32_t logical = (lane % C::CPR) ^ gm_swz<C::CPR>(r);
+    uint32_t src = r < (uint32_t)C::BM ? r : r - C::BM;
+    if (SW && r >= (uint32_t)C::BM)
+        src = 16 * (src / 32) + 8 * (src / 16 % 2) + src % 8;
+    return src * row_bytes + 16 * logical;
+}
+
+// The tile's products: K slices stream through a ring of ST LDS stages by
+// buffer-load DMA, ST - 1 slices ahead of the MFMAs.  What bounds it: the
+// MFMAs (at the clock the power limit leaves) for 256 x 256, whose two stages
+// fill the LDS; for tiles of which a CU runs one, the DMA's latency, which a
+// ring of three or four stages covers.  The hand-over from slice to slice
+// sits before the last k-step's MFMAs (their operands already in registers)
+// and the next slice's first operand reads after it, so that neither the
+// barrier nor the LDS latency leaves the matrix cores idle.  Measured against
+// two stages with the hand-over between slices and 2-4 tile sizes by rule
+// (us, before -> after): 4096 x 4096 x 4096 108.4 -> 102.3 (1343 TFLOP/s); T
+// = 1371, 1024-wide layer: q/k/v 16.1 -> 14.5, o 10.8 -> 10.1, gate/up 25.3
+// -> 21.4, down 18.5 -> 15.4; T = 37: 6.1 -> 5.3, 9.2 -> 7.0, 12.6 -> 5.3,
+// 12.4 -> 8.9; T = 600, 4096-wide: 51 -> 32, 45 -> 26, 194 -> 120, 130 -> 74.
 template <typename C, bool SW>
 __global__ __launch_bounds__(C::THREADS, C::MINB) void gemm_kernel(GemmArgs g) {
-    constexpr int IM = C::IM, JN = C::JN;
-    static_assert(!SW || JN == 2, "the SwiGLU pairing needs two column blocks per wave");
+    constexpr int IM = C::IM, JN = C::JN, BK = C::BK, KS = C::KS, ST = C::ST;
     const uint32_t T = g.T, N = g.N;
     const uint16_t* __restrict__ x = g.x;
     // One array per stage (A rows, then B rows), so that the compiler can
-    // tell the stage being read from the one the DMA is filling.
-    __shared__ __align__(1024) uint16_t s_0[C::A_ELEMS + C::B_ELEMS];
-    __shared__ __align__(1024) uint16_t s_1[C::A_ELEMS + C::B_ELEMS];
+    // tell the stage being read from those the DMA is filling.
+    constexpr int STAGE = C::A_ELEMS + C::B_ELEMS;
+    __shared__ __align__(1024) uint16_t s_0[STAGE];
+    __shared__ __align__(1024) uint16_t s_1[STAGE];
+    __shared__ __align__(1024) uint16_t s_2[ST > 2 ? STAGE : 8];
+    __shared__ __align__(1024) uint16_t s_3[ST > 3 ? STAGE : 8];
     // Output tiles run over the segments' rows stacked, each segment
     // starting on a tile boundary.
     const uint32_t n_tm = gm_out_tiles<C, SW>(g);
@@ -363,16 +424,11 @@ __global__ __launch_bounds__(C::THREADS, C::MINB) void gemm_kernel(GemmArgs g) {
     uint16_t* __restrict__ y = pick3(g.y, seg);
     const uint32_t t0 = tile.tt * C::BM, m0 = tm * TILE_N;
     const uint32_t row_bytes = 2 * N;
-    const auto ra = make_rsrc(x + (size_t)t0 * N, min((uint32_t)C::BM, T - t0) * row_bytes);
-    const uint32_t b_rows = min(TILE_N, M - m0);
-    const auto rb = make_rsrc(pick3(g.w, seg) + (size_t)m0 * N, b_rows * row_bytes);
-    const auto rb_up = make_rsrc(pick3(g.w, SW ? 1 : seg) + (size_t)m0 * N, b_rows * row_bytes);
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int wr = wave / C::WGN, wc = wave % C::WGN;
 
     // Operand read offsets (elements) inside a stage for block 0, per
     // k-step; block i adds 32 i rows.
-    constexpr int BK = C::BK, KS = C::KS;
     int a_off[KS], b_off[KS];
 #pragma unroll
     for (int s = 0; s < KS; ++s) {
@@ -389,83 +445,141 @@ __global__ __launch_bounds__(C::THREADS, C::MINB) void gemm_kernel(GemmArgs g) {
 #pragma unroll
             for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.0f;
 
+    // Every wave issues DMAS instructions per slice, which the vmcnt waits
+    // count on: where BLOCKS is not a multiple of the waves, the surplus
+    // ones load one of the last two blocks again (the same bytes to the same
+    // place, and of the same kind, gate or up: WAVES and BLOCKS are even).
     const uint32_t nk = N / BK;
-    auto dma_slice = [&](uint32_t kt, uint16_t* st) __attribute__((always_inline)) {
-        gm_dma<C::WAVES, C::A_DMA, C::CPR>(ra, row_bytes, kt * BK * 2, st);
-        if constexpr (!SW) {
-            gm_dma<C::WAVES, C::B_DMA, C::CPR>(rb, row_bytes, kt * BK * 2, st + C::A_ELEMS);
-        } else {
-            // One DMA instruction fills 64 / CPR rows inside one 32-row block.
-            const int wave_s = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t wave_s = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    uint32_t d_off[C::DMAS], d_blk[C::DMAS];
 #pragma unroll
-            for (int j = 0; j < C::B_DMA; ++j) {
-                const int blk = wave_s + C::WAVES * j;
-                const uint32_t r = (64 / C::CPR) * blk + lane / C::CPR;  // tile row
-                const uint32_t b32 = ((64 / C::CPR) * blk) / 32;         // its 32-row block
-                const uint32_t src = 32 * (b32 / 2) + r % 32;            // row of gate / up
-                const uint32_t logical = (lane % C::CPR) ^ gm_swz<C::CPR>(r);
-                dma16(b32 & 1 ? rb_up : rb, st + C::A_ELEMS + 512 * blk,
-                      src * row_bytes + kt * BK * 2 + 16 * logical);
-            }
-        }
+    for (int j = 0; j < C::DMAS; ++j) {
+        const uint32_t blk = wave_s + C::WAVES * j;
+        d_blk[j] = blk < (uint32_t)C::BLOCKS ? blk : C::BLOCKS - 2 + blk % 2;
+        d_off[j] = gm_dma_offset<C, SW>(d_blk[j], lane, row_bytes);
+    }
+    // The next slice to load: its first column in A and in this wave's part
+    // of B, and the bytes from there to the tile's end.  Past the last slice
+    // (the ring runs in whole rounds of ST) the ranges are empty: the loads
+    // give zeros, which add nothing.
+    const uint16_t* pa = x + (size_t)t0 * N;
+    const uint16_t* pb = pick3(g.w, seg) + (size_t)m0 * N;
+    if (SW && wave_s % 2) pb = g.w[1] + (size_t)m0 * N;
+    uint32_t a_left = min((uint32_t)C::BM, T - t0) * row_bytes;
+    uint32_t b_left = min(TILE_N, M - m0) * row_bytes;
+    uint32_t k_left = nk;
+    auto dma_slice = [&](uint16_t* st) __attribute__((always_inline)) {
+        const auto ra = make_rsrc(pa, k_left ? a_left : 0);
+        const auto rb = make_rsrc(pb, k_left ? b_left : 0);
+#pragma unroll
+        for (int j = 0; j < C::DMAS; ++j)
+            dma16(C::WAVES * j < C::A_BLOCKS ? ra : rb, st + 512 * d_blk[j], d_off[j]);
     };
-    // Step kt: wait for slice kt, barrier, start slice kt + 1 into the stage
-    // step kt - 1 read, then KS k-steps of MFMAs from stage kt % 2.
-    auto step = [&](uint32_t kt, const uint16_t* cur, uint16_t* nxt) __attribute__((always_inline)) {
-        __builtin_amdgcn_s_waitcnt(kWaitVmcnt0);
-        // The reads of step kt - 1 have all been consumed by its MFMAs; the
-        // memory clobber keeps this step's reads and DMA below the barrier.
-        asm volatile("s_barrier" ::: "memory");
-        if (kt + 1 < nk) dma_slice(kt + 1, nxt);
-        // Operands of k-step s + 1 are read while the MFMAs of k-step s run
-        // (two register sets).
-        bf16x8_t a[2][IM], b[2][JN];
-        auto read = [&](int s) __attribute__((always_inline)) {
+    auto next_slice = [&]() __attribute__((always_inline)) {
+        pa += BK;
+        pb += BK;
+        a_left -= 2 * BK;
+        b_left -= 2 * BK;
+        k_left -= k_left != 0;
+    };
+    // Operands of k-step s + 1 are read while the MFMAs of k-step s run (two
+    // register sets; KS is even, so a slice starts on set 0).
+    bf16x8_t a[2][IM], b[2][JN];
+    auto read = [&](const uint16_t* st, int s) __attribute__((always_inline)) {
 #pragma unroll
-            for (int i = 0; i < IM; ++i)
-                a[s & 1][i] = as_bf16x8(*reinterpret_cast<const uint4*>(cur + a_off[s] + 32 * BK * i));
+        for (int i = 0; i < IM; ++i)
+            a[s & 1][i] = as_bf16x8(*reinterpret_cast<const uint4*>(st + a_off[s] + 32 * BK * i));
+#pragma unroll
+        for (int j = 0; j < JN; ++j)
+            b[s & 1][j] = as_bf16x8(*reinterpret_cast<const uint4*>(st + b_off[s] + 32 * BK * j));
+    };
+    auto mfmas = [&](int s) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < IM; ++i)
 #pragma unroll
             for (int j = 0; j < JN; ++j)
-                b[s & 1][j] = as_bf16x8(*reinterpret_cast<const uint4*>(cur + b_off[s] + 32 * BK * j));
-        };
-        read(0);
-#pragma unroll
-        for (int s = 0; s < KS; ++s) {
-            if (s < KS - 1) read(s + 1);
-#pragma unroll
-            for (int i = 0; i < IM; ++i)
-#pragma unroll
-                for (int j = 0; j < JN; ++j)
-                    acc[i][j] = mfma32x32x16(b[s & 1][j], a[s & 1][i], acc[i][j]);  // W rows first
-        }
-        // Schedule: reads of k-steps 0 and 1, then each k-step's MFMAs
-        // followed by the reads of the k-step after the next.
-        __builtin_amdgcn_sched_group_barrier(0x100, 2 * (IM + JN), 0);
-#pragma unroll
-        for (int s = 0; s < KS; ++s) {
-            __builtin_amdgcn_sched_group_barrier(0x008, IM * JN, 0);
-            if (s < KS - 2) __builtin_amdgcn_sched_group_barrier(0x100, IM + JN, 0);
-        }
+                acc[i][j] = mfma32x32x16(b[s & 1][j], a[s & 1][i], acc[i][j]);  // W rows first
     };
-    dma_slice(0, s_0);
-    for (uint32_t kt = 0; kt < nk; kt += 2) {
-        step(kt, s_0, s_1);
-        if (kt + 1 < nk) step(kt + 1, s_1, s_0);
+    // Slice kt, in `cur`, its first operands already in registers: the MFMAs
+    // of k-steps 0 .. KS - 2; then, with the last k-step's operands in
+    // registers too, the hand-over (this wave's reads of cur and its part of
+    // slice kt + 1 have landed, then every wave's have), the first operand
+    // reads of slice kt + 1 and the DMA of slice kt + ST into cur, all spread
+    // over the MFMAs of the last k-step.
+    constexpr int DMAS = C::DMAS;
+    auto step = [&](uint16_t* cur, const uint16_t* nxt) __attribute__((always_inline)) {
+#pragma unroll
+        for (int s = 0; s < KS - 1; ++s) {
+            read(cur, s + 1);
+            mfmas(s);
+            __builtin_amdgcn_sched_group_barrier(0x100, IM + JN, 0);
+            __builtin_amdgcn_sched_group_barrier(0x008, IM * JN, 0);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_s_waitcnt(wait_vmcnt_lgkm0((ST - 2) * DMAS));
+        asm volatile("s_barrier" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+        read(nxt, 0);
+        dma_slice(cur);
+        mfmas(KS - 1);
+        __builtin_amdgcn_sched_group_barrier(0x100, IM + JN, 0);
+#pragma unroll
+        for (int k = 0; k < IM * JN; ++k) {
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x020, (DMAS + IM * JN - 1) / (IM * JN), 0);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        next_slice();
+    };
+    dma_slice(s_0);
+    next_slice();
+    dma_slice(s_1);
+    next_slice();
+    if constexpr (ST > 2) {
+        dma_slice(s_2);
+        next_slice();
     }
+    if constexpr (ST > 3) {
+        dma_slice(s_3);
+        next_slice();
+    }
+    __builtin_amdgcn_s_waitcnt(wait_vmcnt_lgkm0((ST - 1) * DMAS));
+    asm volatile("s_barrier" ::: "memory");
+    read(s_0, 0);
+    for (uint32_t kt = 0; kt < nk; kt += ST) {
+        step(s_0, s_1);
+        if constexpr (ST == 2) {
+            step(s_1, s_0);
+        } else if constexpr (ST == 3) {
+            step(s_1, s_2);
+            step(s_2, s_0);
+        } else {
+            step(s_1, s_2);
+            step(s_2, s_3);
+            step(s_3, s_0);
+        }
+    }
+    // The ring is free for the epilogue once every wave's last reads and
+    // (empty) DMA are done.
+    __builtin_amdgcn_s_waitcnt(kWaitVmLgkm0);
+    asm volatile("s_barrier" ::: "memory");
 
     // Block (i, j), W rows first: lane l value v is output column
-    // 32 (JN wc + j) + 8 (v / 4) + 4 (l / 32) + v % 4 of token row
-    // 32 (IM wr + i) + l % 32, so v / 4 picks four consecutive outputs of one
-    // token.  Each wave stages its bf16 results (rows of OUTC outputs) in
-    // its part of the ring slot the last step did not read, R token blocks
-    // at a time, and writes whole 16-byte chunks of token rows.
-    constexpr int OUTC = SW ? 32 : 32 * JN;  // a wave's output columns
-    constexpr int CR = OUTC / 8;             // 16-byte chunks per staged row
-    constexpr int AREA = (C::A_ELEMS + C::B_ELEMS) / C::WAVES;  // elements per wave
-    constexpr int R = IM < AREA / (32 * OUTC) ? IM : AREA / (32 * OUTC);
-    static_assert(R >= 1 && (CR == 4 || CR == 8 || CR == 12), "epilogue staging");
+    // 32 (JN wc + j) + 8 (v / 4) + 4 (l / 32) + v % 4 (SW: gate v = 8 q + u and
+    // up 8 q + 4 + u of column 16 (JN wc + j) + 8 q + 4 (l / 32) + u) of token
+    // row 32 (IM wr + i) + l % 32, so v / 4 picks four consecutive outputs of
+    // one token.  Each wave stages its bf16 results (rows of OUTC outputs) in
+    // its part of the first stage, R token blocks at a time, and writes whole
+    // 16-byte chunks of token rows.
+    constexpr int OUTC = SW ? 16 * JN : 32 * JN;  // a wave's output columns
+    constexpr int CR = OUTC / 8;                  // 16-byte chunks per staged row
+    constexpr int AREA = STAGE / C::WAVES / 64 * 64;  // elements per wave
+    constexpr int FIT = CR == 2 ? 2 : AREA / (32 * OUTC);
+    constexpr int R = IM < FIT ? IM : FIT;
+    static_assert(32 * R * OUTC <= AREA, "epilogue area");
+    static_assert(R >= 1 && (CR == 2 || CR == 4 || CR == 6 || CR == 8 || CR == 12), "epilogue staging");
     constexpr int PER_LANE = 32 * R * CR / 64;  // chunks a lane moves per round (R CR is even)
-    uint16_t* const area = (nk % 2 ? s_1 : s_0) + wave * AREA;
+    uint16_t* const area = s_0 + wave * AREA;
     const uint32_t col0 = m0 + OUTC * wc;
     const bool residual = !SW && g.residual;
     // Whole 16-byte stores need every row start 16-byte aligned.
@@ -492,19 +606,20 @@ __global__ __launch_bounds__(C::THREADS, C::MINB) void gemm_kernel(GemmArgs g) {
             if (ii >= nb) break;
             const int i = r0 + ii, t = 32 * ii + (lane & 31);
 #pragma unroll
-            for (int j = 0; j < OUTC / 32; ++j)
+            for (int j = 0; j < JN; ++j)
 #pragma unroll
-                for (int q = 0; q < 4; ++q) {
+                for (int q = 0; q < (SW ? 2 : 4); ++q) {
                     float e[4];
 #pragma unroll
                     for (int u = 0; u < 4; ++u) {
                         if constexpr (SW)
-                            e[u] = swiglu1(bf16_to_f32(f32_to_bf16(acc[i][0][4 * q + u])),
-                                           bf16_to_f32(f32_to_bf16(acc[i][1][4 * q + u])));
+                            e[u] = swiglu1(bf16_to_f32(f32_to_bf16(acc[i][j][8 * q + u])),
+                                           bf16_to_f32(f32_to_bf16(acc[i][j][8 * q + 4 + u])));
                         else
                             e[u] = acc[i][j][4 * q + u];
                     }
-                    const int pc = ep_chunk<CR>(4 * j + q, t), h = (lane >> 5) ^ ep_swap<CR>(t);
+                    const int pc = ep_chunk<CR>((SW ? 2 : 4) * j + q, t);
+                    const int h = (lane >> 5) ^ ep_swap<CR>(t);
                     ep_write(area + t * OUTC + 8 * pc + 4 * h, pack_bf16x2(e[0], e[1]),
                              pack_bf16x2(e[2], e[3]));
                 }
@@ -556,13 +671,6 @@ uint32_t gemm_tiles(const GemmArgs& g) {
     return ((g.T + C::BM - 1) / C::BM) * gm_out_tiles<C, SW>(g);
 }
 
-template <typename C>
-bool gemm_whole(const GemmArgs& g) {
-    for (int sg = 0; sg < g.nseg; ++sg)
-        if (g.rows[sg] % C::BN) return false;
-    return true;
-}
-
 template <typename C, bool SW = false>
 hipError_t gemm_launch(const GemmArgs& g, hipStream_t stream) {
     gemm_kernel<C, SW><<<gemm_tiles<C, SW>(g), C::THREADS, 0, stream>>>(g);
@@ -578,6 +686,39 @@ int gemm_cus() {
         return n;
     }();
     return cus;
+}
+
+template <typename C, bool SW>
+float gemm_cost(const GemmArgs& g, uint32_t cus) {
+    const float tiles = (float)gemm_tiles<C, SW>(g);
+    const float rounds = ceilf(tiles / cus), u = tiles / (rounds * cus);
+    const float slices = (float)(g.N / kGmBK);
+    return C::COST.fixed + rounds * (C::COST.round + slices * (C::COST.slice + C::COST.load * u));
+}
+
+// The configuration of least modelled cost.  Every one sums K in the same
+// MFMA order, so the choice does not change a result bit.
+template <bool SW>
+hipError_t gemm_pick_launch(const GemmArgs& g, hipStream_t stream) {
+    const uint32_t cus = (uint32_t)gemm_cus();
+    hipError_t (*best)(const GemmArgs&, hipStream_t) = nullptr;
+    float least = 0.0f;
+    auto consider = [&](float cost, hipError_t (*launch)(const GemmArgs&, hipStream_t)) {
+        if (best == nullptr || cost < least) {
+            least = cost;
+            best = launch;
+        }
+    };
+    consider(gemm_cost<GmMini, SW>(g, cus), gemm_launch<GmMini, SW>);
+    consider(gemm_cost<GmSix, SW>(g, cus), gemm_launch<GmSix, SW>);
+    consider(gemm_cost<GmFlat, SW>(g, cus), gemm_launch<GmFlat, SW>);
+    consider(gemm_cost<GmDeep, SW>(g, cus), gemm_launch<GmDeep, SW>);
+    consider(gemm_cost<GmTall, SW>(g, cus), gemm_launch<GmTall, SW>);
+    consider(gemm_cost<GmHalf, SW>(g, cus), gemm_launch<GmHalf, SW>);
+    consider(gemm_cost<GmWide, SW>(g, cus), gemm_launch<GmWide, SW>);
+    consider(gemm_cost<GmBroad, SW>(g, cus), gemm_launch<GmBroad, SW>);
+    consider(gemm_cost<GmLarge, SW>(g, cus), gemm_launch<GmLarge, SW>);
+    return best(g, stream);
 }
 
 }  // namespace
@@ -611,31 +752,7 @@ hipError_t launch_batch_proj_bf16(const uint16_t* W, const uint16_t* x, uint16_t
 }
 
 hipError_t launch_gemm(const GemmArgs& g, hipStream_t stream) {
-    // The largest tile whose tiles alone fill every CU once; 64 x 64 below that.
-    const uint32_t cus = (uint32_t)gemm_cus();
-    if (g.swiglu) {
-        // Tiles with two column blocks per wave: 256 x 256 when they fill the
-        // CUs; 192 x 128 when 128 x 128 would need a second round and these do
-        // not; else 128 x 128.
-        if (gemm_tiles<GmLarge, true>(g) >= cus) return gemm_launch<GmLarge, true>(g, stream);
-        if (gemm_tiles<GmSmall, true>(g) > 2 * cus && gemm_tiles<GmTall, true>(g) <= 2 * cus)
-            return gemm_launch<GmTall, true>(g, stream);
-        return gemm_launch<GmSmall, true>(g, stream);
-    }
-    if (gemm_tiles<GmLarge>(g) >= cus) return gemm_launch<GmLarge>(g, stream);
-    // 128 x 128 tiles that would put two on some CUs and not on others: one
-    // 192 x 128 tile per CU when those fit (the stacked q/k/v projections of
-    // a 1371-token prompt: 15.7 against 16.5 us).
-    if (gemm_tiles<GmSmall>(g) > cus && gemm_tiles<GmTall>(g) <= cus) return gemm_launch<GmTall>(g, stream);
-    // 128 x 128 tiles that overflow the two resident workgroups per CU leave
-    // a second, mostly idle round: 128 x 192 tiles, when they fit one round
-    // (and every segment is whole tiles of 192), take it in one.
-    if (gemm_tiles<GmSmall>(g) > 2 * cus && gemm_tiles<GmMid>(g) <= 2 * cus &&
-        gemm_whole<GmMid>(g))
-        return gemm_launch<GmMid>(g, stream);
-    if (gemm_tiles<GmSmall>(g) >= cus) return gemm_launch<GmSmall>(g, stream);
-    if (g.N % GmMini::BK == 0) return gemm_launch<GmMini>(g, stream);
-    return gemm_launch<GmMini64>(g, stream);
+    return g.swiglu ? gemm_pick_launch<true>(g, stream) : gemm_pick_launch<false>(g, stream);
 }
 
 }  // namespace tiattn
