@@ -126,12 +126,19 @@ def _ptr(t) -> Optional[int]:
 
 def _stream(stream) -> Optional[int]:
     """hipStream_t handle: an int, a torch.cuda.Stream, or None for torch's
-    current stream on the current device."""
+    current stream on the current device.
+
+    torch.cuda.current_stream() builds a Stream object on every call, 3.2 us
+    of a one-kernel call's 7.4 us on the host (3.7 us of it HIP's launch); the
+    same handle comes in 0.2 us from the lookup underneath, once torch has
+    initialised the device (before that, its own error or initialisation)."""
     if isinstance(stream, int):
         return stream
     import torch
 
     if stream is None:
+        if torch.cuda.is_initialized():
+            return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
         stream = torch.cuda.current_stream()
     return int(stream.cuda_stream)
 
