@@ -177,6 +177,37 @@ def test_fused_equals_unfused_composition(dev):
     H.check_bar(a, b, "fused vs unfused", max_abs=1e-2, mean_abs=2e-4)
 
 
+@pytest.mark.parametrize("s,hq,hkv,d,o_is", [
+    (1, 4, 2, 128, None), (31, 16, 8, 64, "q"), (33, 6, 3, 128, "k"), (127, 2, 2, 64, "k"),
+    (1023, 32, 8, 128, "k"), (1371, 16, 8, 128, None), (1371, 16, 8, 128, "q")])
+def test_fused_prefill_prepared_q(dev, s, hq, hkv, d, o_is):
+    """Lengths whose attention runs on a prepared Q held in Os: bit for bit
+    the norm/rope kernel on Q and K followed by the plain prefill, also with
+    Os the raw Q's buffer or one that starts with the raw K."""
+    print(f"[fused] prepared Q S={s} {hq}/{hkv} D={d} o_is={o_is}", flush=True)
+    qb, kb, vb, gq, gk = config4_inputs(s, hq, hkv, d, seed=6)
+    q, k, v = H.to_dev_bf16(qb, dev), H.to_dev_bf16(kb, dev), H.to_dev_bf16(vb, dev)
+    g1, g2 = H.to_dev_bf16(gq, dev), H.to_dev_bf16(gk, dev)
+    f = torch.empty(d // 2, dtype=torch.float32, device=dev)
+    attn.precompute_freq_f32(f, d, 1e6)
+    table = torch.empty((s, d // 2, 2), dtype=torch.float32, device=dev)
+    attn.rope_cos_sin_f32(table, f, s, d)
+    qn, kn, exp = torch.empty_like(q), torch.empty_like(k), torch.empty_like(q)
+    attn.qk_norm_rope_bf16(q, g1, qn, f, 1e-6, s, hq, d)
+    attn.qk_norm_rope_bf16(k, g2, kn, f, 1e-6, s, hkv, d)
+    attn.flash_attention_v1_bf16(qn, kn, v, exp, hq, hkv, d, s)
+    o = q if o_is == "q" else torch.full_like(q, -3.0)
+    if o_is == "k":
+        raw = o.view(-1)[:k.numel()]
+        raw.copy_(k.view(-1))
+        k = raw
+    k_out = torch.empty_like(kn)
+    attn.prefill_qknorm_rope_attention_bf16(q, k, v, o, k_out, g1, g2, table, 1e-6, hq, hkv, d, s)
+    H.sync()
+    assert np.array_equal(H.from_dev_bf16(k_out), H.from_dev_bf16(kn))
+    assert np.array_equal(H.from_dev_bf16(o), H.from_dev_bf16(exp))
+
+
 def test_fused_prefill_head_pairs_ragged_rows(dev):
     """The fused entry at a length where the head-pair 128-row kernel is
     chosen (S = 4100, 32/8: 33 query tiles x 16 pairs, two rounds of the

@@ -121,6 +121,9 @@ struct PrefillProblem {
                               // 3: split over keys, GQA head pairs per workgroup (1 for odd groups),
                               // 4: 128-row tiles, GQA head pairs per workgroup (2 for odd groups)
 };
+// fused_q problems (Q raw, transformed on load) run the 128-row kernel only:
+// for those prefill_uses_split() says, prepare Q first.  q may be o: a
+// workgroup reads an item's Q rows before it writes the same rows of o.
 hipError_t launch_prefill(const PrefillProblem& p, hipStream_t stream);
 // Whether launch_prefill takes the split-over-keys kernel for this problem.
 bool prefill_uses_split(const PrefillProblem& p);

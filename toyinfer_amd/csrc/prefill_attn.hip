@@ -573,7 +573,7 @@ __device__ __forceinline__ uint32_t sk_item_index(uint32_t round, uint32_t g, ui
     return round * G + m;
 }
 
-template <int D, bool FUSED>
+template <int D>
 __global__ __launch_bounds__(kPfThreads, 2) void prefill_splitkv_kernel(PrefillProblem p,
                                                                         float scale_log2,
                                                                         uint32_t n_items) {
@@ -621,12 +621,10 @@ __global__ __launch_bounds__(kPfThreads, 2) void prefill_splitkv_kernel(PrefillP
         load_v(t);
     };
     const int st_row = lane / P::CPR, st_c = lane % P::CPR;  // this lane's chunk of a tile row
-    // The first tile's loads go out before anything waits on Q (after the
-    // fused prologue, whose loads need the registers, when FUSED).
+    // The first tile's loads go out before anything waits on Q.
     bf16x8_t qf[P::KSTEPS];
-    if constexpr (FUSED) load_q<D, FUSED>(qf, p, it.q0 + ql, it.h, kg);
     if ((uint32_t)wave < it.n_tiles) load(wave);
-    if constexpr (!FUSED) load_q<D, FUSED>(qf, p, it.q0 + ql, it.h, kg);
+    load_q<D, false>(qf, p, it.q0 + ql, it.h, kg);
 
     while (true) {
         const uint32_t q0 = it.q0, qq = q0 + ql, n_tiles = it.n_tiles;
@@ -730,18 +728,17 @@ __global__ __launch_bounds__(kPfThreads, 2) void prefill_splitkv_kernel(PrefillP
         }
 
         // The next item's first tile and Q loads go out now and land while
-        // this item's partials are merged.  (With FUSED the grid holds every
-        // item: its Q prologue would not fit beside the merge's registers.)
+        // this item's partials are merged.
         ++round;
         const uint32_t nxt = sk_item_index(round, blockIdx.x, gridDim.x);
-        const bool more = !FUSED && nxt < n_items;
+        const bool more = nxt < n_items;
         const uint32_t h = it.h;
         if (more) {
             it = sk_item(p, nxt, group, n_qt);
             rk = make_rsrc(p.k + (int64_t)it.kvh * D, kv_bytes);
             rv = make_rsrc(p.v + (int64_t)it.kvh * D, kv_bytes);
             if ((uint32_t)wave < it.n_tiles) load(wave);
-            load_q<D, FUSED>(qf, p, it.q0 + ql, it.h, kg);
+            load_q<D, false>(qf, p, it.q0 + ql, it.h, kg);
         }
 
         // Merge the four waves' partials of the 32 rows.
@@ -1055,7 +1052,7 @@ __device__ __forceinline__ void sp_merge_stream(f32x16_t (&o)[DB], float4* area,
     else asm volatile("; merge, stream 3");
 }
 
-template <int D, bool FUSED>
+template <int D>
 __global__ __launch_bounds__(kSpThreads, 1) void prefill_splitkv_pair_kernel(PrefillProblem p,
                                                                              float scale_log2,
                                                                              uint32_t n_items) {
@@ -1112,7 +1109,7 @@ __global__ __launch_bounds__(kSpThreads, 1) void prefill_splitkv_pair_kernel(Pre
     };
     bf16x8_t qf[P::KSTEPS];
     if ((uint32_t)stream < it.n_tiles) dma(stream, s_a);
-    load_q<D, FUSED>(qf, p, it.q0 + ql, it.h0 + sub, kg);
+    load_q<D, false>(qf, p, it.q0 + ql, it.h0 + sub, kg);
 
     while (true) {
         const uint32_t q0 = it.q0, qq = q0 + ql, n_tiles = it.n_tiles;
@@ -1217,18 +1214,17 @@ __global__ __launch_bounds__(kSpThreads, 1) void prefill_splitkv_pair_kernel(Pre
         }
         // Every wave is done with both buffers (the last step's barrier): the
         // next item's first tiles go to s_a and its Q to registers, landing
-        // while this item merges in s_b.  (With FUSED the grid holds every
-        // item: its Q prologue would not fit beside the merge's registers.)
+        // while this item merges in s_b.
         ++round;
         const uint32_t nxt = sk_item_index(round, blockIdx.x, gridDim.x);
-        const bool more = !FUSED && nxt < n_items;
+        const bool more = nxt < n_items;
         const uint32_t h = it.h0 + sub;
         if (more) {
             it = sp_item(p, nxt, group, n_qt);
             k_head = p.k + (int64_t)it.kvh * D;
             v_head = p.v + (int64_t)it.kvh * D;
             if ((uint32_t)stream < it.n_tiles) dma(stream, s_a);
-            load_q<D, FUSED>(qf, p, it.q0 + ql, it.h0 + sub, kg);
+            load_q<D, false>(qf, p, it.q0 + ql, it.h0 + sub, kg);
         }
 
         // Merge: the four streams' partials of each head in two exchange
@@ -1291,52 +1287,55 @@ template <int D>
 hipError_t launch_pairs(const PrefillProblem& p, float sl2, uint32_t items, uint32_t slots,
                         hipStream_t st) {
     const dim3 grid(min(items, slots));
-    hipLaunchKernelGGL((prefill_splitkv_pair_kernel<D, false>), grid, dim3(kSpThreads), 0, st, p,
+    hipLaunchKernelGGL((prefill_splitkv_pair_kernel<D>), grid, dim3(kSpThreads), 0, st, p,
                        sl2, items);
     return hipGetLastError();
 }
 
-template <int D, bool FUSED>
-hipError_t launch_t(const PrefillProblem& p, hipStream_t st) {
-    const uint32_t n_qtiles = (p.s + kPfBM - 1) / kPfBM;
-    const float sl2 = kLog2e / sqrtf((float)D);
-    const bool split = prefill_uses_split(p);
-    // Short sequences with an even GQA group take the pair kernel when asked
-    // (variant 3), or by shape when it has more items than the device holds
-    // workgroups of it at D = 128: with fewer it leaves CUs idle, and at
-    // D = 64 a tile's work is too small for its per-step barrier and merge
-    // (measured on MI355X: S = 1371, 16/8 heads, 21.3 -> 18.7 us at D = 128,
-    // 12.1 -> 12.5 us at D = 64; S = 512: 9.1 -> 10.8 us).  The fused Q
-    // prologue stays with the single-head kernel.
-    if (!FUSED && split && (p.hq / p.hkv) % 2 == 0 && p.variant != 1) {
+template <int D>
+hipError_t launch_split(const PrefillProblem& p, float sl2, hipStream_t st) {
+    // An even GQA group takes the pair kernel when asked (variant 3), or by
+    // shape when it has more items than the device holds workgroups of it at
+    // D = 128: with fewer it leaves CUs idle, and at D = 64 a tile's work is
+    // too small for its per-step barrier and merge (measured on MI355X: S =
+    // 1371, 16/8 heads, 21.3 -> 18.7 us at D = 128, 12.1 -> 12.5 us at D = 64;
+    // S = 512: 9.1 -> 10.8 us).
+    if ((p.hq / p.hkv) % 2 == 0 && p.variant != 1) {
         static int cache[64];
         const uint32_t items = ((p.s + kSkBM - 1) / kSkBM) * p.hkv * (p.hq / p.hkv / 2);
-        const uint32_t slots = resident_slots(prefill_splitkv_pair_kernel<D, false>, kSpThreads, 1, cache);
+        const uint32_t slots = resident_slots(prefill_splitkv_pair_kernel<D>, kSpThreads, 1, cache);
         if (p.variant == 3 || (D == 128 && items > slots)) return launch_pairs<D>(p, sl2, items, slots, st);
     }
-    if (split) {
-        const uint32_t items = ((p.s + kSkBM - 1) / kSkBM) * p.hq;
-        static int cache[64];
-        const dim3 grid(FUSED ? items : min(items, resident_slots(prefill_splitkv_kernel<D, FUSED>, kPfThreads, 2, cache)));
-        hipLaunchKernelGGL((prefill_splitkv_kernel<D, FUSED>), grid, dim3(kPfThreads), 0, st, p,
-                           sl2, items);
-    } else {
-        // Head pairs per workgroup when the GQA group is even and the pair
-        // grid is at least two rounds of the device (measured on MI355X,
-        // 32/8 heads: S = 8192 490 -> 479 us, S = 4096 150 -> 143 us, but
-        // S = 2048, one round, 50 -> 58 us).
-        static int cache[64];
-        const uint32_t pair_wgs = n_qtiles * (p.hq / 2);
-        const bool even = (p.hq / p.hkv) % 2 == 0;
-        if (even && (p.variant == 4 ||
-                     (p.variant == 0 && pair_wgs >= 2 * resident_slots(prefill_kernel<D, FUSED, true>, 512, 1, cache)))) {
-            hipLaunchKernelGGL((prefill_kernel<D, FUSED, true>), dim3(pair_wgs), dim3(512), 0, st, p, sl2);
-        } else {
-            hipLaunchKernelGGL((prefill_kernel<D, FUSED, false>), dim3(n_qtiles * p.hq), dim3(kPfThreads), 0,
-                               st, p, sl2);
-        }
-    }
+    static int cache[64];
+    const uint32_t items = ((p.s + kSkBM - 1) / kSkBM) * p.hq;
+    const dim3 grid(min(items, resident_slots(prefill_splitkv_kernel<D>, kPfThreads, 2, cache)));
+    hipLaunchKernelGGL((prefill_splitkv_kernel<D>), grid, dim3(kPfThreads), 0, st, p, sl2, items);
     return hipGetLastError();
+}
+
+template <int D, bool FUSED>
+hipError_t launch_rows(const PrefillProblem& p, float sl2, hipStream_t st) {
+    // Head pairs per workgroup when the GQA group is even and the pair
+    // grid is at least two rounds of the device (measured on MI355X,
+    // 32/8 heads: S = 8192 490 -> 479 us, S = 4096 150 -> 143 us, but
+    // S = 2048, one round, 50 -> 58 us).
+    const uint32_t n_qtiles = (p.s + kPfBM - 1) / kPfBM;
+    static int cache[64];
+    const uint32_t pair_wgs = n_qtiles * (p.hq / 2);
+    const bool even = (p.hq / p.hkv) % 2 == 0;
+    if (even && (p.variant == 4 ||
+                 (p.variant == 0 && pair_wgs >= 2 * resident_slots(prefill_kernel<D, FUSED, true>, 512, 1, cache))))
+        hipLaunchKernelGGL((prefill_kernel<D, FUSED, true>), dim3(pair_wgs), dim3(512), 0, st, p, sl2);
+    else
+        hipLaunchKernelGGL((prefill_kernel<D, FUSED, false>), dim3(n_qtiles * p.hq), dim3(kPfThreads), 0, st, p, sl2);
+    return hipGetLastError();
+}
+
+template <int D>
+hipError_t launch_t(const PrefillProblem& p, hipStream_t st) {
+    const float sl2 = kLog2e / sqrtf((float)D);
+    if (p.fused_q) return launch_rows<D, true>(p, sl2, st);
+    return prefill_uses_split(p) ? launch_split<D>(p, sl2, st) : launch_rows<D, false>(p, sl2, st);
 }
 
 }  // namespace
@@ -1347,8 +1346,7 @@ bool prefill_uses_split(const PrefillProblem& p) {
 }
 
 hipError_t launch_prefill(const PrefillProblem& p, hipStream_t stream) {
-    if (p.d == 64) return p.fused_q ? launch_t<64, true>(p, stream) : launch_t<64, false>(p, stream);
-    return p.fused_q ? launch_t<128, true>(p, stream) : launch_t<128, false>(p, stream);
+    return p.d == 64 ? launch_t<64>(p, stream) : launch_t<128>(p, stream);
 }
 
 }  // namespace tiattn
