@@ -22,6 +22,7 @@ from toyinfer_amd import attn, synth
 pytestmark = pytest.mark.gpu
 
 SENTINEL = 0x7F11
+SENTINEL_F = 7.0  # for buffers held as bf16 values
 
 
 def order_slack(w_f32, x_f32):
@@ -277,3 +278,58 @@ def test_gemm_swiglu_equals_projections_then_swiglu(dev, T, hid, M):
     attn.batch_swiglu_bf16x2(gate, up, ref, T, M)
     torch.cuda.synchronize()
     assert torch.equal(out.view(torch.int16), ref.view(torch.int16))
+
+
+# The K-split kernel of few tokens: token tiles of 16, 32 and 48 with
+# remainders, output tiles of 16 and 32 with remainders, fewer chunks than
+# waves, uneven shares of K, and both sides of the line to the ring GEMM
+# (T rows <= 327680, T <= 320).
+@pytest.mark.parametrize("T,M,N", [(5, 1, 64), (5, 17, 576), (16, 15, 512), (17, 130, 3072),
+                                   (48, 1024, 2048), (49, 33, 4160), (80, 4096, 1024),
+                                   (81, 4096, 1024), (320, 1024, 1024), (321, 1000, 1024),
+                                   (9, 12289, 128), (37, 8853, 192)])
+def test_batch_proj_few_tokens(dev, T, M, N):
+    print(f"[step] few tokens T={T} M={M} N={N}", flush=True)
+    g = torch.Generator(device=dev).manual_seed(40)
+    w = (torch.randn((M, N), generator=g, device=dev) * 0.03).to(torch.bfloat16)
+    x = torch.randn((T, N), generator=g, device=dev).to(torch.bfloat16)
+    buf = torch.full((T * M + 9,), SENTINEL_F, dtype=torch.bfloat16, device=dev)
+    attn.batch_gemv_proj_bf16(w, x, buf, T, M, N)
+    # One rounding to bf16 and fp32 sums in any order.
+    ref = x.double() @ w.double().t()
+    slack = (x.double().abs() @ w.double().abs().t()) * 2.0 ** -20
+    H.sync()
+    err = (buf[:T * M].view(T, M).double() - ref).abs()
+    assert bool((err <= ref.abs() * 2.0 ** -8 + slack).all()), f"max err {float(err.max())}"
+    assert bool((buf[T * M:] == SENTINEL_F).all())
+
+
+@pytest.mark.parametrize("T,hid,rows", [(128, 512, (4096, 1024, 130)), (81, 1024, (4096, 4095, 33)),
+                                        (5, 64, (1, 16, 33)), (320, 1024, (1024, 1025, 7))])
+def test_few_token_segments_and_epilogues(dev, T, hid, rows):
+    """Stacks whose segments lie on both sides of the line, the residual form
+    and gate/up with SwiGLU equal the separate operations bit for bit."""
+    print(f"[step] few-token segments T={T} hid={hid} rows={rows}", flush=True)
+    g = torch.Generator(device=dev).manual_seed(41)
+    x = torch.randn((T, hid), generator=g, device=dev).to(torch.bfloat16)
+    ws = [(torch.randn((r, hid), generator=g, device=dev) * 0.05).to(torch.bfloat16) for r in rows]
+    old = [torch.randn((T, r), generator=g, device=dev).to(torch.bfloat16) for r in rows]
+    ys, res = [torch.empty_like(o) for o in old], [o.clone() for o in old]
+    attn.gemm_segments_bf16(x, T, hid, ws, ys, rows)
+    attn.gemm_segments_bf16(x, T, hid, ws, res, rows, residual=True)
+    for w, y, o, s, r in zip(ws, ys, old, res, rows):
+        ref = torch.empty_like(y)
+        attn.batch_gemv_proj_bf16(w, x, ref, T, r, hid)
+        added = (o.float() + ref.float()).to(torch.bfloat16)
+        H.sync()
+        assert torch.equal(y.view(torch.int16), ref.view(torch.int16)), f"rows {r}"
+        assert torch.equal(s.view(torch.int16), added.view(torch.int16)), f"residual, rows {r}"
+        if r % 2 == 0:
+            up = torch.flip(w, (0,)).contiguous()
+            out, gu = torch.empty_like(y), torch.empty_like(y)
+            attn.gemm_swiglu_bf16(x, T, hid, w, up, r, out)
+            attn.batch_gemv_proj_bf16(up, x, gu, T, r, hid)
+            exp = torch.empty_like(y)
+            attn.batch_swiglu_bf16x2(ref, gu, exp, T, r)
+            H.sync()
+            assert torch.equal(out.view(torch.int16), exp.view(torch.int16)), f"swiglu, rows {r}"

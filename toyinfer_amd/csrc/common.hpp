@@ -22,6 +22,7 @@ constexpr float kLog2e = 1.4426950408889634f;
 // s_waitcnt immediates (gfx9 encoding: vmcnt[3:0] and [15:14], expcnt[6:4],
 // lgkmcnt[11:8]); the fields not named are left at their maximum (no wait).
 constexpr int kWaitVmcnt0 = 0x0F70;  // vmcnt(0)
+constexpr int kWaitLgkm0 = 0xC07F;    // lgkmcnt(0)
 constexpr int kWaitVmLgkm0 = 0x0070;  // vmcnt(0) lgkmcnt(0)
 constexpr int wait_vmcnt_lgkm0(int n) { return 0x0070 | (n & 15) | (n >> 4) << 14; }
 constexpr int wait_vmcnt(int n) { return 0x0F70 | (n & 15) | (n >> 4) << 14; }  // vmcnt(n), n < 64

@@ -201,6 +201,20 @@ struct GemmArgs {
     bool swiglu = false;
 };
 hipError_t launch_gemm(const GemmArgs& g, hipStream_t stream);
+// The same for a few tokens, with K split over the waves of a workgroup
+// (another summation order).  launch_gemm sends each segment of `rows`
+// outputs there by T and rows alone, so that a stacked segment, a gate/up
+// pair and the projection by itself give the same bits.  The line: the ring
+// GEMM's 64 x 64 tiles fill the CUs from about T rows = 2^20 on, and each of
+// its tiles reads a quarter of the bytes per output (measured, weights from
+// HBM, ring -> K split, us: M = 1024, N = 3072, T = 256 16.9 -> 9.4; M = 2560,
+// N = 4096, T = 128 20.9 -> 13.1, T = 256 20.8 -> 20.6; M = 4096, N = 4096, T =
+// 64 21.6 -> 13.5, T = 100 19.7 -> 18.9, T = 192 21.3 -> 23.2; gate/up of 9728,
+// N = 2560, T = 37 29.7 -> 34.2).
+inline bool proj_uses_skinny(uint32_t T, uint32_t rows) {
+    return T <= 320 && (uint64_t)T * rows <= 5u << 16;
+}
+hipError_t launch_gemm_skinny(const GemmArgs& g, hipStream_t stream);
 
 // ------------------------------------------------- fused decode projections
 // One token: y = W * f(x) with f = RMSNorm(x; norm_w, eps) when norm_w is set,

@@ -752,7 +752,22 @@ hipError_t launch_batch_proj_bf16(const uint16_t* W, const uint16_t* x, uint16_t
 }
 
 hipError_t launch_gemm(const GemmArgs& g, hipStream_t stream) {
-    return g.swiglu ? gemm_pick_launch<true>(g, stream) : gemm_pick_launch<false>(g, stream);
+    if (g.swiglu)
+        return proj_uses_skinny(g.T, g.rows[0]) ? launch_gemm_skinny(g, stream)
+                                                : gemm_pick_launch<true>(g, stream);
+    // The segments of each kind in one launch.
+    GemmArgs part[2] = {g, g};
+    part[0].nseg = part[1].nseg = 0;
+    for (int s = 0; s < g.nseg; ++s) {
+        GemmArgs& p = part[proj_uses_skinny(g.T, g.rows[s])];
+        p.w[p.nseg] = g.w[s];
+        p.y[p.nseg] = g.y[s];
+        p.rows[p.nseg++] = g.rows[s];
+    }
+    hipError_t e = hipSuccess;
+    if (part[0].nseg) e = gemm_pick_launch<false>(part[0], stream);
+    if (e == hipSuccess && part[1].nseg) e = launch_gemm_skinny(part[1], stream);
+    return e;
 }
 
 }  // namespace tiattn
