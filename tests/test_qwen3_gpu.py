@@ -122,6 +122,30 @@ def test_decode_vs_oracle(dev, graph):
     m.close()
 
 
+@pytest.mark.parametrize("hq,hkv,d,msl", [(1, 1, 64, 64), (12, 2, 128, 64), (6, 1, 64, 98560),
+                                          (7, 1, 64, 64), (16, 1, 128, 64), (7, 1, 64, 98560)])
+def test_decode_group_sizes_vs_oracle(dev, hq, hkv, d, msl):
+    """The decode attention's row prologue at its edges: 1 and 6 query heads
+    per KV head (32 lanes a row), 7 and 16 (D/16 lanes), both split rules (the
+    long cache has more 128-row slices than splits), new rows on either side
+    of a 32-row chunk boundary."""
+    print(f"[step] qwen3 decode groups {hq}/{hkv} d={d} msl={msl}", flush=True)
+    cfg = dict(TINY, num_q_heads=hq, num_kv_heads=hkv, head_dim=d, max_seq_len=msl)
+    host, dw = make_weights(cfg, dev, seed=57)
+    T, steps = 30, 4
+    ids = prompt(T, cfg["vocab_size"], seed=58)
+    m = qwen3.Qwen3(qwen3.Config(**cfg), dw)
+    H.sync()
+    m.prefill(ids_dev(ids, dev), T)
+    ref = oracle.Qwen3Reference(cfg, host)
+    ref.forward(ids, 0)
+    for s in range(steps):
+        m.decode(1, s % 2 == 1)
+        toks = m.tokens_host(T + s + 2)
+        check_logits(m.logits_host(), ref.forward([toks[T + s]], T + s), f"step {s}")
+    m.close()
+
+
 def test_graph_equals_direct_launches(dev):
     """Two models, same weights and prompt: 3 + 5 graph replays (one capture)
     vs 8 directly launched steps give the same tokens and identical logits."""

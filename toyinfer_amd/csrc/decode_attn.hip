@@ -49,10 +49,10 @@ constexpr int kDecMaxHeads = 16;                          // MFMA columns = quer
 __device__ __forceinline__ uint32_t seq_length(const DecodeProblem& p, uint32_t b) {
     if (p.len_mode == kLenHost) return p.len_host;
     if (p.len_mode == kLenDevice) {
-        const uint32_t L = p.len_dev[b];
+        const uint32_t L = scalar_load(p.len_dev + b);
         return L < p.len_cap ? L : p.len_cap;
     }
-    const uint32_t pos = p.len_dev[0];
+    const uint32_t pos = scalar_load(p.len_dev);
     return (pos < p.len_cap ? pos : p.len_cap - 1) + 1;
 }
 
@@ -119,15 +119,21 @@ __device__ __forceinline__ CompatLayout compat_layout(const DecodeProblem& p,
     return c;
 }
 
+// Prologue rows of 32 lanes in a workgroup: up to six query heads per KV head
+// plus k and v (Qwen3-0.6B: 0.662 -> 0.647 ms per decode step against rows of
+// D / 16 lanes, which larger groups keep: 18 rows do not fit 32 lanes each).
+constexpr int kFewRows = 8;
+
 // Workgroup blockIdx.x takes a fixed slice [t_begin, t_end) of the positions
 // (split_range), its wave w the 32-row chunks w, w+4, ... of that slice.
 // PRO: the engine's form with the token's q/k norm + RoPE and cache-row
 // writes folded in (DecodePrologue).
 // COMPAT: the reference-contract pass (B = 1, partials in the score rows,
 // raw scores stored when compat_layout says so).
+// FEW (PRO only): up to kFewRows - 2 query heads per KV head.
 // FIXED (PRO only): p.slice_rows == 128, split s owns rows [128 s, 128 s +
 // 128) whatever the length.
-template <int D, bool PRO, bool COMPAT = false, bool FIXED = false>
+template <int D, bool PRO, bool COMPAT = false, bool FIXED = false, bool FEW = false>
 __device__ __forceinline__ void decode_split_body(const DecodeProblem& p,
                                                   const DecodePartials& part_in, float scale_log2,
                                                   const DecodePrologue& pro) {
@@ -143,12 +149,23 @@ __device__ __forceinline__ void decode_split_body(const DecodeProblem& p,
                                                                             : LDS_BYTES_O];
     __shared__ float s_ml[kDecWaves][kDecMaxHeads][2];
 
+    if constexpr (PRO) {
+        fetch_args(p.q, p.k, p.v, p.hq, p.hkv, p.len_dev, p.len_cap, p.splits, part_in.ml,
+                   part_in.o, part_in.ml_head, part_in.o_head, part_in.o_split, scale_log2, p.group,
+                   p.head_groups);
+        fetch_args(pro.q_w, pro.k_raw, pro.k_w, pro.v_raw, pro.rope, pro.k_cache, pro.v_cache,
+                   pro.eps);
+    }
+    // PRO takes its length from len_dev (kLenDevice), requested here by a
+    // scalar load (the wait for it leaves the vector loads in flight).
+    uint32_t len_pro = 0;
+    if constexpr (PRO) len_pro = scalar_load(p.len_dev);
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int n = lane & 15, g = lane >> 4;
-    const uint32_t group = p.hq / p.hkv;
-    const uint32_t n_hg = (group + kDecMaxHeads - 1) / kDecMaxHeads;
-    const uint32_t kvh = blockIdx.y / n_hg, hgi = blockIdx.y % n_hg;
-    const uint32_t b = blockIdx.z;
+    const uint32_t group = p.group, n_hg = p.head_groups;
+    const uint32_t kvh = n_hg == 1 ? blockIdx.y : blockIdx.y / n_hg;
+    const uint32_t hgi = n_hg == 1 ? 0 : blockIdx.y % n_hg;
+    const uint32_t b = PRO ? 0 : blockIdx.z;
     const uint32_t h0 = kvh * group + hgi * kDecMaxHeads;
     const uint32_t nh = min((uint32_t)kDecMaxHeads, group - hgi * kDecMaxHeads);
     const int64_t bh0 = (int64_t)b * p.hq + h0;
@@ -189,7 +206,19 @@ __device__ __forceinline__ void decode_split_body(const DecodeProblem& p,
     int pmode = -1;  // -1: no prologue row in this lane
     NormRopeIn pin;
     uint4 pro_a, pro_b;  // the lane's two output chunks of its prologue row
-    if constexpr (PRO) {
+    // FEW: rows of 32 lanes, q heads in rows 0 .. nh-1, then k and v.
+    constexpr int kFewV = kFewRows - 1, kFewK = kFewRows - 2;
+    const int frow = threadIdx.x / 32, fc = threadIdx.x % 32;
+    const int frow_lds = frow == kFewK ? kNewK : frow == kFewV ? kNewV : frow;
+    NormRopePairs<D> fin;
+    if constexpr (PRO && FEW) {
+        const bool is_k = frow == kFewK, is_v = frow == kFewV;
+        const uint16_t* src = is_k   ? pro.k_raw + (int64_t)kvh * D
+                              : is_v ? pro.v_raw + (int64_t)kvh * D
+                                     : p.q + (bh0 + ((uint32_t)frow < nh ? frow : 0)) * D;
+        fin = norm_rope_pairs_load<D>(src, is_k ? pro.k_w : pro.q_w, pro.rope, fc);
+        __builtin_amdgcn_sched_barrier(0);
+    } else if constexpr (PRO) {
         // Every lane runs one unconditional load sequence (per-lane sources;
         // lanes without a row re-read q row 0, the v row loads weights and
         // angles it does not use): loads under a branch would make the
@@ -210,7 +239,10 @@ __device__ __forceinline__ void decode_split_body(const DecodeProblem& p,
     // Normalise + rotate the rows (row kNewV is a copy) into LDS; needs no
     // length.
     auto pro_compute = [&]() {
-        if (pmode >= 0) {
+        if constexpr (FEW) {
+            norm_rope_pairs_compute<D>(fin, pro.eps, frow == kFewV);
+            if (frow >= kFewK || (uint32_t)frow < nh) fin.put(s_pro + frow_lds * D, fc);
+        } else if (pmode >= 0) {
             norm_rope_compute<D>(pin, true, pro.eps, 0, pmode, &pro_a, &pro_b);
             *reinterpret_cast<uint4*>(s_pro + prow * D + 8 * pc) = pro_a;
             *reinterpret_cast<uint4*>(s_pro + prow * D + 8 * pc + D / 2) = pro_b;
@@ -222,17 +254,10 @@ __device__ __forceinline__ void decode_split_body(const DecodeProblem& p,
     // its rows clamped to the cache (len_cap); rows at or past the length are
     // masked and their V zeroed in the loop.  The prologue rows are computed
     // meanwhile.
-    // PRO takes its length from len_dev (kLenDevice); FIXED requests it
-    // behind the chunk (a scalar load: its wait leaves the vector loads in
-    // flight) and uses it after the prologue arithmetic.
-    uint32_t len_pro = 0;
     if constexpr (FIXED) {
         load_rows(blockIdx.x * kDecIterRows + wave * kDecWaveRows, p.len_cap);
         __builtin_amdgcn_sched_barrier(0);
-        len_pro = p.len_dev[b];
         pro_compute();
-    } else if constexpr (PRO) {
-        len_pro = p.len_dev[b];
     }
 
     const uint32_t L = PRO ? min(len_pro, p.len_cap) : seq_length(p, b);
@@ -324,7 +349,11 @@ __device__ __forceinline__ void decode_split_body(const DecodeProblem& p,
     // them), then Q^T from LDS.
     if constexpr (PRO) {
         if constexpr (!FIXED) pro_compute();
-        if (pmode >= 0 && prow >= kNewK && has_new && hgi == 0) {
+        if (FEW) {
+            if (frow >= kFewK && has_new)
+                fin.put((frow == kFewK ? pro.k_cache : pro.v_cache) + ((int64_t)pos * p.hkv + kvh) * D,
+                        fc);
+        } else if (pmode >= 0 && prow >= kNewK && has_new && hgi == 0) {
             uint16_t* crow = (prow == kNewK ? pro.k_cache : pro.v_cache) +
                              ((int64_t)pos * p.hkv + kvh) * D;
             *reinterpret_cast<uint4*>(crow + 8 * pc) = pro_a;
@@ -494,12 +523,12 @@ __global__ __launch_bounds__(256, 3) void decode_split_compat_kernel(DecodeProbl
 
 // The engine's single-sequence grid (splits x Hkv workgroups) is far below
 // one per CU, so the register budget is not cut for occupancy.
-template <int D, bool FIXED>
+template <int D, bool FIXED, bool FEW>
 __global__ __launch_bounds__(256, 1) void decode_split_pro_kernel(DecodeProblem p,
                                                                   DecodePartials part,
                                                                   float scale_log2,
                                                                   DecodePrologue pro) {
-    decode_split_body<D, true, false, FIXED>(p, part, scale_log2, pro);
+    decode_split_body<D, true, false, FIXED, FEW>(p, part, scale_log2, pro);
 }
 
 // Merge the splits of one (sequence, q-head) in a 256-thread block.  The
@@ -680,6 +709,7 @@ __global__ __launch_bounds__(kSliceDims * kSliceGroups) void decode_combine_slic
     constexpr int U = 4;
     __shared__ float s_acc[kSliceGroups][kSliceDims];
     __shared__ float s_ml[kSliceGroups][2];
+    fetch_args(part.ml, part.o, part.ml_head, part.o_head, part.o_split, splits, o, o_f32);
     const int dl = threadIdx.x % kSliceDims, sg = threadIdx.x / kSliceDims;
     const int64_t bh = blockIdx.x;
     const int d = blockIdx.y * kSliceDims + dl;
@@ -743,7 +773,7 @@ __global__ __launch_bounds__(kCombineThreads) void decode_finalize_compat_kernel
     }
     const float inv = den > 0.0f ? 1.0f / den : 0.0f;
     const float mref = M == -INFINITY ? 0.0f : M;
-    const uint32_t kvh = h / (p.hq / p.hkv);
+    const uint32_t kvh = h / p.group;
     float* srow = score + (int64_t)h * msl;
     for (uint32_t t = threadIdx.x; t < msl; t += blockDim.x) {
         float val = 0.0f;
@@ -766,27 +796,41 @@ __global__ __launch_bounds__(kCombineThreads) void decode_finalize_compat_kernel
     }
 }
 
+DecodeProblem grouped(DecodeProblem p) {
+    p.group = p.hq / p.hkv;
+    p.head_groups = decode_head_groups(p.group);
+    return p;
+}
+
 template <int D>
-hipError_t launch_split_t(const DecodeProblem& p, const DecodePartials& part, hipStream_t st) {
-    const uint32_t group = p.hq / p.hkv;
-    const dim3 grid(p.splits, p.hkv * decode_head_groups(group), p.batch);
+hipError_t launch_split_t(const DecodeProblem& problem, const DecodePartials& part,
+                          hipStream_t st) {
+    const DecodeProblem p = grouped(problem);
+    const dim3 grid(p.splits, p.hkv * p.head_groups, p.batch);
     const float sl2 = kLog2e / sqrtf((float)D);
     hipLaunchKernelGGL((decode_split_kernel<D>), grid, dim3(256), 0, st, p, part, sl2);
     return hipGetLastError();
 }
 
 template <int D>
-hipError_t launch_split_pro_t(const DecodeProblem& p, const DecodePartials& part,
+hipError_t launch_split_pro_t(const DecodeProblem& problem, const DecodePartials& part,
                               const DecodePrologue& pro, hipStream_t st) {
-    const uint32_t group = p.hq / p.hkv;
-    const dim3 grid(p.splits, p.hkv * decode_head_groups(group), 1);
+    const DecodeProblem p = grouped(problem);
+    const dim3 grid(p.splits, p.hkv * p.head_groups, 1);
     const float sl2 = kLog2e / sqrtf((float)D);
-    if (p.slice_rows != 0)
-        hipLaunchKernelGGL((decode_split_pro_kernel<D, true>), grid, dim3(256), 0, st, p, part, sl2,
-                           pro);
+    const bool few = p.group <= (uint32_t)kFewRows - 2;
+    if (p.slice_rows != 0 && few)
+        hipLaunchKernelGGL((decode_split_pro_kernel<D, true, true>), grid, dim3(256), 0, st, p,
+                           part, sl2, pro);
+    else if (p.slice_rows != 0)
+        hipLaunchKernelGGL((decode_split_pro_kernel<D, true, false>), grid, dim3(256), 0, st, p,
+                           part, sl2, pro);
+    else if (few)
+        hipLaunchKernelGGL((decode_split_pro_kernel<D, false, true>), grid, dim3(256), 0, st, p,
+                           part, sl2, pro);
     else
-        hipLaunchKernelGGL((decode_split_pro_kernel<D, false>), grid, dim3(256), 0, st, p, part,
-                           sl2, pro);
+        hipLaunchKernelGGL((decode_split_pro_kernel<D, false, false>), grid, dim3(256), 0, st, p,
+                           part, sl2, pro);
     return hipGetLastError();
 }
 
@@ -842,6 +886,8 @@ __device__ __forceinline__ float2 stash_get(const uint16_t* o_row) {
 template <int D>
 __global__ __launch_bounds__(kCombineThreads) void decode_compat_merge_kernel(
     DecodeProblem p, DecodePartials part, float* o_buffer, uint16_t* o) {
+    fetch_args(p.d, p.len_mode, p.len_dev, p.len_host, p.len_cap, p.splits, part.ml, part.o,
+               part.ml_head, part.o_head, part.o_split, o_buffer, o);
     const uint32_t h = blockIdx.x;
     const CompatLayout cl = compat_layout(p, part, seq_length(p, 0));
     float M, den;
@@ -866,9 +912,11 @@ __global__ __launch_bounds__(256) void decode_compat_score_kernel(
     __shared__ __align__(16) uint16_t s_tile[kDecWaves][kDecWaveRows * D];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int n = lane & 15, g = lane >> 4;
-    const uint32_t group = p.hq / p.hkv;
-    const uint32_t n_hg = (group + kDecMaxHeads - 1) / kDecMaxHeads;
-    const uint32_t kvh = blockIdx.y / n_hg, hgi = blockIdx.y % n_hg;
+    fetch_args(p.q, p.k, p.hq, p.hkv, p.d, p.len_mode, p.len_dev, p.len_host, p.len_cap, p.splits,
+               p.group, p.head_groups, score, msl, o, scale_log2);
+    const uint32_t group = p.group, n_hg = p.head_groups;
+    const uint32_t kvh = n_hg == 1 ? blockIdx.y : blockIdx.y / n_hg;
+    const uint32_t hgi = n_hg == 1 ? 0 : blockIdx.y % n_hg;
     const uint32_t h0 = kvh * group + hgi * kDecMaxHeads;
     const uint32_t nh = min((uint32_t)kDecMaxHeads, group - hgi * kDecMaxHeads);
     const uint32_t L = seq_length(p, 0);
@@ -994,9 +1042,10 @@ hipError_t launch_decode_split(const DecodeProblem& p, const DecodePartials& par
     return launch_split_t<128>(p, part, stream);
 }
 
-hipError_t launch_decode_split_compat(const DecodeProblem& p, const DecodePartials& part,
+hipError_t launch_decode_split_compat(const DecodeProblem& problem, const DecodePartials& part,
                                       hipStream_t stream) {
-    const dim3 grid(p.splits, p.hkv * decode_head_groups(p.hq / p.hkv), 1);
+    const DecodeProblem p = grouped(problem);
+    const dim3 grid(p.splits, p.hkv * p.head_groups, 1);
     const float sl2 = kLog2e / sqrtf((float)p.d);
     if (p.d == 64)
         hipLaunchKernelGGL((decode_split_compat_kernel<64>), grid, dim3(256), 0, stream, p, part, sl2);
@@ -1045,9 +1094,10 @@ hipError_t launch_decode_combine(const DecodeProblem& p, const DecodePartials& p
     return hipGetLastError();
 }
 
-hipError_t launch_decode_finalize_compat(const DecodeProblem& p, const DecodePartials& part,
+hipError_t launch_decode_finalize_compat(const DecodeProblem& problem, const DecodePartials& part,
                                          float* score, uint32_t msl, float* o_buffer,
                                          uint16_t* o, hipStream_t stream) {
+    const DecodeProblem p = grouped(problem);
     const dim3 grid(p.hq);
     const float sl2 = kLog2e / sqrtf((float)p.d);
     if (p.splits >= 2) {
@@ -1059,7 +1109,7 @@ hipError_t launch_decode_finalize_compat(const DecodeProblem& p, const DecodePar
             hipLaunchKernelGGL(decode_compat_merge_kernel<128>, grid, dim3(kCombineThreads), 0,
                                stream, p, part, o_buffer, o);
         const dim3 sgrid((msl + kDecIterRows - 1) / kDecIterRows,
-                         p.hkv * decode_head_groups(p.hq / p.hkv));
+                         p.hkv * p.head_groups);
         if (p.d == 64)
             hipLaunchKernelGGL(decode_compat_score_kernel<64>, sgrid, dim3(64 * kDecWaves), 0, stream,
                                p, score, msl, o, sl2);

@@ -200,25 +200,42 @@ __global__ __launch_bounds__(kDgThreads) void decode_gemv_kernel(DecodeGemvArgs 
 // (4-12 MB of weights): 3.4-4.9 us per projection, against 4-6 us for the
 // block-cooperative kernel below; 16-wave workgroups on 32-48 CUs stream the
 // same matrices from HBM at under half the rate (8.5 us for 4 MB).  The
-// residual row is read at the start, with the weights; the weight rows carry
-// the non-temporal hint (read once per step: 0.729 -> 0.666 ms per
-// Qwen3-0.6B decode step together with the lm-head's).
+// residual row is read at the start, by every lane (left to the compiler it is
+// read where it is added, another trip to memory at the end); the input goes
+// out ahead of the weights, whose flight then covers the norm; and the
+// arguments come in one round.  Those three: 0.675 -> 0.664 ms per Qwen3-0.6B
+// decode step.  The weight rows carry the non-temporal hint (read once per
+// step: 0.729 -> 0.666 ms together with the lm-head's).  Repeated from one
+// graph with weights from HBM, a launch takes 2.8 (o), 3.1 (down), 3.2 (q/k/v)
+// and 4.0 us (gate/up); with the weights in L2 2.2-3.1, an empty kernel 1.7.
 constexpr int kDwWaves = 4;
 
 template <int RPW, int NCH, bool NORM, int EPI>
 __global__ __launch_bounds__(64 * kDwWaves) void decode_gemv_wave_kernel(DecodeGemvArgs a) {
     constexpr int NR = EPI == kDgSwiglu ? 2 * RPW : RPW;
+    if constexpr (EPI == kDgPlain)
+        fetch_args(a.x, NORM ? a.norm_w : a.x, a.eps, a.n, a.nseg, a.w[0], a.w[1], a.w[2], a.y[0],
+                   a.y[1], a.y[2], a.rows[0], a.rows[1], a.rows[2]);
+    else
+        fetch_args(a.x, NORM ? a.norm_w : a.x, a.eps, a.n, a.w[0], EPI == kDgSwiglu ? a.w[1] : a.x,
+                   a.y[0], a.rows[0]);
     const int lane = threadIdx.x & 63;
     const uint32_t wave =
         __builtin_amdgcn_readfirstlane(blockIdx.x * kDwWaves + (threadIdx.x >> 6));
     const uint32_t N = a.n;
     uint32_t r0 = wave * RPW;
-    const uint32_t spans[3] = {(a.rows[0] + RPW - 1) / RPW * RPW, (a.rows[1] + RPW - 1) / RPW * RPW,
-                               (a.rows[2] + RPW - 1) / RPW * RPW};
-    const int seg = segment_of(spans, a.nseg, r0);
-    const uint32_t seg_rows = pick3(a.rows, seg);
-    const uint16_t* const seg_w = pick3(a.w, seg);
-    uint16_t* const seg_y = pick3(a.y, seg);
+    uint32_t seg_rows = a.rows[0];
+    const uint16_t* seg_w = a.w[0];
+    uint16_t* seg_y = a.y[0];
+    if constexpr (EPI == kDgPlain) {  // the others have one segment
+        const uint32_t spans[3] = {(a.rows[0] + RPW - 1) / RPW * RPW,
+                                   (a.rows[1] + RPW - 1) / RPW * RPW,
+                                   (a.rows[2] + RPW - 1) / RPW * RPW};
+        const int seg = segment_of(spans, a.nseg, r0);
+        seg_rows = pick3(a.rows, seg);
+        seg_w = pick3(a.w, seg);
+        seg_y = pick3(a.y, seg);
+    }
     if (r0 >= seg_rows) return;  // a grid's last waves may have no rows
     const uint32_t nrows = min((uint32_t)RPW, seg_rows - r0);
     const uint32_t row_bytes = 2 * N;
@@ -227,6 +244,19 @@ __global__ __launch_bounds__(64 * kDwWaves) void decode_gemv_wave_kernel(DecodeG
     if constexpr (EPI == kDgSwiglu) rw[1] = make_rsrc(a.w[1] + (size_t)r0 * N, nrows * row_bytes);
     const __amdgpu_buffer_rsrc_t rx = make_rsrc(a.x, row_bytes);
     uint4 wv[NR][NCH], xv[NCH], gv[NCH];
+    // Unconditional (rows past the end read 0): under a branch its latency
+    // would be paid again at the end.
+    uint16_t res = 0;
+    if constexpr (EPI == kDgResidual)
+        res = __builtin_amdgcn_raw_buffer_load_b16(make_rsrc(seg_y + r0, 2 * nrows), 2 * lane, 0, 0);
+    // The input first: its sum of squares is taken while the rows arrive.
+#pragma unroll
+    for (int k = 0; k < NCH; ++k) {
+        const uint32_t off = 16 * (lane + 64 * k);
+        xv[k] = buf_load16(rx, off);
+        if constexpr (NORM) gv[k] = buf_load16(make_rsrc(a.norm_w, row_bytes), off);
+    }
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int k = 0; k < NCH; ++k) {
         // Chunks past the row's end read zeros: their offset is moved past
@@ -236,11 +266,8 @@ __global__ __launch_bounds__(64 * kDwWaves) void decode_gemv_wave_kernel(DecodeG
 #pragma unroll
         for (int r = 0; r < NR; ++r)
             wv[r][k] = buf_load16_nt(rw[r / RPW], in ? (r % RPW) * row_bytes + off : 0x80000000u);
-        xv[k] = buf_load16(rx, off);
-        if constexpr (NORM) gv[k] = buf_load16(make_rsrc(a.norm_w, row_bytes), off);
     }
-    uint16_t res = 0;
-    if (EPI == kDgResidual && (uint32_t)lane < nrows) res = seg_y[r0 + lane];
+    __builtin_amdgcn_sched_barrier(0);
 
     if constexpr (NORM) {
         float ss = 0.0f;
@@ -279,17 +306,17 @@ __global__ __launch_bounds__(64 * kDwWaves) void decode_gemv_wave_kernel(DecodeG
         v = lane == r ? sum[r] : v;
         if constexpr (EPI == kDgSwiglu) u = lane == r ? sum[RPW + r] : u;
     }
-    if ((uint32_t)lane < nrows) {
-        const uint32_t m = r0 + lane;
-        if constexpr (EPI == kDgPlain) {
-            seg_y[m] = f32_to_bf16(v);
-        } else if constexpr (EPI == kDgResidual) {
-            seg_y[m] = f32_to_bf16(bf16_to_f32(res) + bf16_round(v));
-        } else {
-            const float g = bf16_round(v), up = bf16_round(u);
-            a.y[0][m] = f32_to_bf16(up * (g * (1.0f / (1.0f + expf(-g)))));
-        }
+    uint32_t out;
+    if constexpr (EPI == kDgPlain) {
+        out = f32_to_bf16(v);
+    } else if constexpr (EPI == kDgResidual) {
+        out = f32_to_bf16(bf16_to_f32(res) + bf16_round(v));
+    } else {
+        const float g = bf16_round(v), up = bf16_round(u);
+        out = f32_to_bf16(up * (g * (1.0f / (1.0f + expf(-g)))));
     }
+    asm volatile("" : "+v"(out));  // computed (and the residual loaded) by every lane
+    if ((uint32_t)lane < nrows) seg_y[r0 + lane] = (uint16_t)out;
 }
 
 template <int RPW, int NCH, bool NORM, int EPI>

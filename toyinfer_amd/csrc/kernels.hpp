@@ -58,6 +58,9 @@ struct DecodeProblem {
     // split s owns cache rows [128 s, 128 s + 128) whatever the length and
     // loads them before the device length arrives.
     uint32_t slice_rows;
+    // Set by the launchers: hq / hkv, and 16-head groups of that.
+    uint32_t group;
+    uint32_t head_groups;
 };
 
 // Split pass: grid (splits, Hkv * head groups, B).

@@ -149,5 +149,80 @@ __device__ __forceinline__ void norm_rope_row(const uint16_t* in, uint16_t* out,
     *reinterpret_cast<uint4*>(out + 8 * c + D / 2) = b;
 }
 
+// A row over 32 lanes, for a workgroup with few rows: lane c holds the D / 64
+// pairs (i, D/2 + i) from i = c D/64 on, so that the loads are narrow (five per
+// lane, up to 16 bytes) and the arithmetic in front of the hand-over is a
+// quarter to an eighth as long as with 8-value chunks (eight 16-byte loads in
+// every lane, whose issue alone held back the cache rows behind them).
+template <int D>
+struct NormRopePairs {
+    static constexpr int P = D / 64;
+    uint32_t x[2], w[2];  // as loaded: P bf16 values of either half of the row and the weights
+    float2 angle[P];
+    float lo[P], hi[P];   // the row's values after the compute phase
+    __device__ __forceinline__ void put(uint16_t* row, int c) const {
+        if constexpr (P == 2) {
+            *reinterpret_cast<uint32_t*>(row + 2 * c) = pack_bf16x2(lo[0], lo[1]);
+            *reinterpret_cast<uint32_t*>(row + D / 2 + 2 * c) = pack_bf16x2(hi[0], hi[1]);
+        } else {
+            row[c] = f32_to_bf16(lo[0]);
+            row[D / 2 + c] = f32_to_bf16(hi[0]);
+        }
+    }
+};
+
+template <int D>
+__device__ __forceinline__ NormRopePairs<D> norm_rope_pairs_load(const uint16_t* in,
+                                                                 const uint16_t* weight,
+                                                                 const float2* angles, int c) {
+    constexpr int P = NormRopePairs<D>::P;
+    NormRopePairs<D> r;
+    auto get = [c](const uint16_t* row) __attribute__((always_inline)) -> uint32_t {
+        if constexpr (P == 2)
+            return *reinterpret_cast<const uint32_t*>(row + 2 * c);
+        else
+            return row[c];
+    };
+    r.x[0] = get(in);
+    r.x[1] = get(in + D / 2);
+    r.w[0] = get(weight);
+    r.w[1] = get(weight + D / 2);
+#pragma unroll
+    for (int k = 0; k < P; ++k) r.angle[k] = angles[P * c + k];
+    return r;
+}
+
+// RMSNorm and RoPE of the row (copy: its values as they are).
+template <int D>
+__device__ __forceinline__ void norm_rope_pairs_compute(NormRopePairs<D>& r, float eps, bool copy) {
+#pragma clang fp contract(off)
+    constexpr int P = NormRopePairs<D>::P;
+    float ss = 0.0f;
+#pragma unroll
+    for (int k = 0; k < P; ++k) {
+        r.lo[k] = k ? bf16_hi(r.x[0]) : bf16_lo(r.x[0]);
+        r.hi[k] = k ? bf16_hi(r.x[1]) : bf16_lo(r.x[1]);
+        ss += r.lo[k] * r.lo[k];
+        ss += r.hi[k] * r.hi[k];
+    }
+    ss += dpp_f32<kDppXor1>(ss);
+    ss += dpp_f32<kDppXor2>(ss);
+    ss += dpp_f32<kDppRowHalfMirror>(ss);
+    ss += dpp_f32<kDppRowMirror>(ss);
+    ss = xor16_sum(ss);
+    const float inv = 1.0f / sqrtf(ss / (float)D + eps);
+#pragma unroll
+    for (int k = 0; k < P; ++k) {
+        const float wl = k ? bf16_hi(r.w[0]) : bf16_lo(r.w[0]);
+        const float wh = k ? bf16_hi(r.w[1]) : bf16_lo(r.w[1]);
+        const float a = bf16_to_f32(f32_to_bf16(r.lo[k] * inv * wl));
+        const float b = bf16_to_f32(f32_to_bf16(r.hi[k] * inv * wh));
+        const float x = r.angle[k].x * a - r.angle[k].y * b;
+        const float y = r.angle[k].x * b + r.angle[k].y * a;
+        r.lo[k] = copy ? r.lo[k] : x;
+        r.hi[k] = copy ? r.hi[k] : y;
+    }
+}
+
 }  // namespace
 }  // namespace tiattn
