@@ -135,3 +135,40 @@ def test_sample_boundaries(dev, V, k):
     rng = np.random.default_rng(V * 7 + k)
     lg = (rng.standard_normal(V) * 2).astype(np.float32)
     check_case(smp, lg, 1.3, k, 0.97, f"boundary V={V} k={k}")
+
+
+def _rows(kind, V, rng):
+    lg = (rng.standard_normal(V) * 2.5).astype(np.float32)
+    if kind == "sorted":        # the top k in one chunk
+        lg.sort()
+    elif kind == "masked":      # five allowed tokens, the rest at -inf
+        keep = rng.choice(V, 5, replace=False)
+        lg[np.setdiff1d(np.arange(V), keep)] = -np.inf
+    elif kind == "lowest":      # the same with the type's lowest value
+        keep = rng.choice(V, 5, replace=False)
+        lg[np.setdiff1d(np.arange(V), keep)] = np.finfo(np.float32).min
+    elif kind == "equal":       # every key a tie
+        lg[:] = 1.5
+    elif kind == "steps":       # more ties at the k-th value than places
+        lg = np.round(lg)
+    elif kind == "strided":     # the largest all with one thread of a chunk
+        lg[7::256] += 20.0
+    return lg
+
+
+@pytest.mark.parametrize("kind", ["normal", "sorted", "masked", "lowest", "equal", "steps",
+                                  "strided"])
+@pytest.mark.parametrize("V,k", [(4095, 20), (4096, 20), (4097, 40), (8191, 21), (151936, 20),
+                                 (151936, 40), (151936, 41), (262144, 2)])
+def test_sample_filter_and_its_fallback(dev, kind, V, k):
+    """The filtered selection at the edges of its rule (k 40 / 41, V 4095 /
+    4096, places 32 / 64), and rows for which it lets through too many keys in
+    a chunk, among the candidates, or in both."""
+    print(f"[step] sample filter {kind} V={V} k={k}", flush=True)
+    smp = Sampler(dev)
+    rng = np.random.default_rng(V + 31 * k)
+    # Equal keys have running sums j / k: 0.93 k is 0.1 or more from any whole
+    # number for every k here, so the cut is at least 0.1 / 41 = 2.4e-3 from a
+    # running sum, far above their rounding (41 steps of 2^-24: 2.4e-6).  (0.95
+    # would put it on one at k = 20 and 40, where either side may round.)
+    check_case(smp, _rows(kind, V, rng), 0.9, k, 0.93, f"{kind} V={V} k={k}")

@@ -22,10 +22,21 @@
 // select (four 8-bit digit passes over per-wave LDS histograms), and writes
 // its top k (keys and indices) to the workspace.  The last workgroup to
 // finish (an agent-scope ticket) runs the same select over the G*k
-// candidates, sorts the k survivors (in one wave's registers for k <= 64,
+// candidates, sorts the k survivors (by rank in one wave for k <= 64,
 // in LDS above), and does the softmax, the top-p cut and the coin walk with
 // lane or block scans.  Ties at the k-th value keep the lowest indices;
 // equal values are ordered by index.
+//
+// What bounds it is that chain of dependent steps, not the 0.6 MB of logits.
+// For small k both selects are therefore replaced by a filter: a lower bound
+// of the k-th largest key (from the 256 threads' own maxima) lets through the
+// top k and a few more, and the final ranking drops those.  Where a filter
+// lets through too many (heavy ties, rows masked to one value) the select
+// runs in its place.  With it, the candidates in four-place loads that are
+// all out at once, and the ranking in place of a bitonic sort (us, V =
+// 151936): k = 2 15.4 -> 11.7, 20 18.2 -> 12.2, 40 21.7 -> 13.2; by select
+// k = 41 21.9 -> 18.6, 64 25.2 -> 20.9, 200 37.1 -> 31.4; V = 8192: k = 20
+// 15.4 -> 11.5, 200 30.4 -> 24.6.
 #include <hip/hip_runtime.h>
 
 #include "../../include/toyinfer_attn.h"
@@ -46,9 +57,27 @@ static_assert(kSpBlocksSmallK * kSpSmallK <= kSpChunk && kSpBlocksLargeK * kSamp
               "candidates fit the per-thread key slots");
 static_assert(kSpBlocksLargeK * kSpChunk >= kSampleMaxVocab, "every chunk fits one workgroup");
 constexpr uint32_t kSpMaxCand = kSpChunk;
+// Filtered selection: k up to kSpFilterK and chunks longer than that.  k keys
+// spread over 256 threads leave about k^2 / 512 of them beside a larger one
+// of the same thread, and the 16-bit bound a few per cent more, so 40 stay
+// within 64 places with room, 20 within 32 and 10 within 16 (each place more
+// is one more for the merge to read: k = 20 12.2 us, 21 12.9); at k = 50 some
+// of the 64 chunks would run over in many calls, which then pay for both forms.
+// Short rows leave most threads without a key to bound with (V = 4095, k = 20:
+// 13.2 us by select, 11.5 filtered at 8192).
+constexpr uint32_t kSpFilterK = 40, kSpFilterMinVocab = 64 * kSpBlocksSmallK;
+static_assert(kSpFilterMinVocab / kSpBlocksSmallK > kSpFilterK, "full chunks exceed k");
+__device__ __forceinline__ uint32_t sp_width(uint32_t n, uint32_t k) {
+    if (k > kSpFilterK || n < kSpFilterMinVocab) return k;
+    return k <= 10 ? 16u : (k <= 20 ? 32u : 64u);
+}
+static_assert(kSpBlocksSmallK * 64 <= kSpMaxCand, "64 places per chunk fit the workspace");
+static_assert(kSpBlocksSmallK % 4 == 0 && kSpBlocksLargeK % 4 == 0 && kSpChunk == 32 * kSpThreads,
+              "the merge loads four places at a time");
 
 // Workspace: [0, 8) argmax key, [8, 12) argmax ticket, [12, 16) sampler
-// ticket, then keys [32][k] and indices [32][k] from byte 256.
+// ticket, then keys [G][width] and indices [G][width] from byte 256 (width:
+// sp_width; places without a candidate hold key 0, index ~0).
 constexpr size_t kSpCandOff = 256;
 
 // Order-preserving map of a float to an unsigned key (larger float, larger key).
@@ -204,6 +233,60 @@ __device__ __forceinline__ uint32_t top_mask(const uint32_t (&key)[kSpPer], cons
     return take;
 }
 
+// A lower bound of the k-th largest valid key of the workgroup: the k-th
+// largest of the threads' maxima, its upper 16 bits (each wave finds them by
+// itself, bit by bit, from all 256 maxima).  0 when fewer than k threads hold
+// a key.
+__device__ __forceinline__ uint32_t bound_kth(const uint32_t (&key)[kSpPer], uint32_t valid, uint32_t k,
+                                              uint32_t* s_max, int slots) {
+    uint32_t mx = 0;
+#pragma unroll
+    for (int j = 0; j < kSpPer; ++j) {
+        if (j >= slots) break;
+        mx = max(mx, valid >> j & 1u ? key[j] : 0u);
+    }
+    s_max[threadIdx.x] = mx;
+    __syncthreads();
+    const uint4 v = reinterpret_cast<const uint4*>(s_max)[threadIdx.x & 63];
+    uint32_t t = 0;
+#pragma unroll
+    for (int bit = 31; bit >= 16; --bit) {
+        const uint32_t c = t | 1u << bit;
+        const uint32_t n = __popcll(__ballot(v.x >= c)) + __popcll(__ballot(v.y >= c)) +
+                           __popcll(__ballot(v.z >= c)) + __popcll(__ballot(v.w >= c));
+        if (n >= k) t = c;
+    }
+    return t;
+}
+
+// Emits the valid keys from that bound on, at least the top k with all ties,
+// if there are at most `room` of them; returns how many there are.
+template <typename F>
+__device__ __forceinline__ uint32_t filter_top(const uint32_t (&key)[kSpPer], uint32_t valid, uint32_t k,
+                                               uint32_t room, uint32_t* s_max, uint32_t* s_cnt,
+                                               int slots, F&& emit) {
+    const uint32_t bound = bound_kth(key, valid, k, s_max, slots);
+    uint32_t take = 0;
+#pragma unroll
+    for (int j = 0; j < kSpPer; ++j) {
+        if (j >= slots) break;
+        take |= (uint32_t)((valid >> j & 1u) && key[j] >= bound) << j;
+    }
+    const uint32_t n = __popc(take);
+    const uint32_t incl = wave_scan_incl(n);
+    uint32_t base = 0;
+    if ((threadIdx.x & 63) == 63) base = atomicAdd(s_cnt, incl);
+    uint32_t slot = read_lane(base, 63) + incl - n;
+    __syncthreads();
+    const uint32_t total = *s_cnt;
+    if (total <= room) {
+#pragma unroll
+        for (int j = 0; j < kSpPer; ++j)
+            if (j < slots && (take >> j & 1u)) emit(slot++, j);
+    }
+    return total;
+}
+
 // Slots 0..k-1 for the set bits of `take` across the workgroup (any order):
 // a wave scan of the per-thread counts and one LDS atomic per wave.
 template <typename F>
@@ -247,9 +330,12 @@ __global__ __launch_bounds__(kSpThreads) void sample_kernel(SampleArgs a) {
     __shared__ __align__(16) uint32_t s_hist[2 * kSpWaves * 256];
     __shared__ uint32_t s_wu[kSpWaves];
     __shared__ float s_wf[kSpWaves];
+    __shared__ __align__(16) uint32_t s_max[kSpThreads];
     __shared__ uint64_t s_top[kSampleMaxK];
+    __shared__ uint64_t s_sorted[64];
     __shared__ float s_acc[kSampleMaxK];
-    __shared__ uint32_t s_res[2], s_cnt;
+    // Emitted keys: by the filter and by the select, of either phase.
+    __shared__ uint32_t s_res[2], s_cnt[4];
     __shared__ bool s_last;
 
     const uint32_t k = a.k, tid = threadIdx.x;
@@ -257,8 +343,10 @@ __global__ __launch_bounds__(kSpThreads) void sample_kernel(SampleArgs a) {
     uint32_t* ticket = reinterpret_cast<uint32_t*>(ws + 12);
     uint32_t* ws_key = reinterpret_cast<uint32_t*>(ws + kSpCandOff);
     const uint32_t G = gridDim.x;
-    uint32_t* ws_idx = ws_key + G * k;
-    if (tid == 0) s_cnt = 0;
+    const uint32_t width = sp_width(a.n, k);
+    const bool filter = width != k;
+    uint32_t* ws_idx = ws_key + G * width;
+    if (tid < 4) s_cnt[tid] = 0;
 
     // Phase 1: this workgroup's chunk, element j*256 + t in thread t's key[j].
     const uint32_t cs = (a.n + G - 1) / G;
@@ -282,26 +370,35 @@ __global__ __launch_bounds__(kSpThreads) void sample_kernel(SampleArgs a) {
             valid |= (uint32_t)(e < m) << j;
         }
     }
-    uint32_t* bk = ws_key + blockIdx.x * k;
-    uint32_t* bi = ws_idx + blockIdx.x * k;
+    uint32_t* bk = ws_key + blockIdx.x * width;
+    uint32_t* bi = ws_idx + blockIdx.x * width;
     if (m <= k) {
         // The whole chunk; key 0 pads (below every key of a non-NaN float).
 #pragma unroll
         for (int j = 0; j < kSpPer; ++j) {
             const uint32_t e = j * kSpThreads + tid;
-            if (e < k) {
+            if (e < width) {
                 bk[e] = e < m ? key[j] : 0u;
                 bi[e] = e < m ? idx[j] : 0xffffffffu;
             }
         }
     } else {
         const int slots = (int)((m + kSpThreads - 1) / kSpThreads);
-        const Sel s = select_kth(key, valid, k, s_hist, slots);
-        const uint32_t take = top_mask(key, idx, valid, s, s_hist, slots);
-        emit_top(take, k, slots, &s_cnt, [&](uint32_t slot, int j) {
+        auto emit = [&](uint32_t slot, int j) {
             bk[slot] = key[j];
             bi[slot] = idx[j];
-        });
+        };
+        uint32_t n = filter ? filter_top(key, valid, k, width, s_max, &s_cnt[0], slots, emit) : ~0u;
+        if (n > width) {
+            const Sel s = select_kth(key, valid, k, s_hist, slots);
+            const uint32_t take = top_mask(key, idx, valid, s, s_hist, slots);
+            emit_top(take, k, slots, &s_cnt[1], emit);
+            n = k;
+        }
+        if (tid >= n && tid < width) {
+            bk[tid] = 0u;
+            bi[tid] = 0xffffffffu;
+        }
     }
     // Every wave waits for its own stores to reach the L2, the barrier joins
     // them, and one agent-scope release (not one per wave) publishes the
@@ -313,30 +410,42 @@ __global__ __launch_bounds__(kSpThreads) void sample_kernel(SampleArgs a) {
         __threadfence();
         s_last = atomicAdd(ticket, 1u) == G - 1;
         if (s_last) __threadfence();
-        s_cnt = 0;
     }
     __syncthreads();
     if (!s_last) return;
 
-    // Phase 2 (last workgroup): the top k of the G*k candidates, as
-    // (key << 32 | ~index) so that one ordering covers the ties.
-    const uint32_t nc = G * k;
+    // Phase 2 (last workgroup): the top k of the G*width candidates, as
+    // (key << 32 | ~index) so that one ordering covers the ties; `found` of
+    // them in s_top, the top k among them.
+    const uint32_t nc = G * width;
+    uint32_t found;
     valid = 0;
+    // Four places per load (nc is a multiple of 4), every load out before the
+    // first is waited for.
+    const int slots = 4 * (int)((nc + 4 * kSpThreads - 1) / (4 * kSpThreads));
+    {
+        const __amdgpu_buffer_rsrc_t rk = make_rsrc(ws_key, nc * 4), ri = make_rsrc(ws_idx, nc * 4);
 #pragma unroll
-    for (int j = 0; j < kSpPer; ++j) {
-        const uint32_t e = j * kSpThreads + tid;
-        const bool v = e < nc && j < (int)((nc + kSpThreads - 1) / kSpThreads);
-        key[j] = v ? ws_key[e] : 0u;
-        idx[j] = v ? ws_idx[e] : 0xffffffffu;
-        valid |= (uint32_t)v << j;
+        for (int j = 0; j < kSpPer; j += 4) {
+            if (j >= slots) break;
+            const uint32_t e = j * kSpThreads + 4 * tid;
+            const uint4 x = buf_load16(rk, 4 * e), y = buf_load16(ri, 4 * e);
+            key[j] = x.x, key[j + 1] = x.y, key[j + 2] = x.z, key[j + 3] = x.w;
+            idx[j] = y.x, idx[j + 1] = y.y, idx[j + 2] = y.z, idx[j + 3] = y.w;
+            valid |= (e < nc ? 15u : 0u) << j;
+        }
     }
     {
-        const int slots = (int)((nc + kSpThreads - 1) / kSpThreads);
-        const Sel s = select_kth(key, valid, k, s_hist, slots);
-        const uint32_t take = top_mask(key, idx, valid, s, s_hist, slots);
-        emit_top(take, k, slots, &s_cnt, [&](uint32_t slot, int j) {
+        auto emit = [&](uint32_t slot, int j) {
             s_top[slot] = ((uint64_t)key[j] << 32) | (uint32_t)~idx[j];
-        });
+        };
+        found = filter ? filter_top(key, valid, k, 64, s_max, &s_cnt[2], slots, emit) : ~0u;
+        if (found > 64) {
+            const Sel s = select_kth(key, valid, k, s_hist, slots);
+            const uint32_t take = top_mask(key, idx, valid, s, s_hist, slots);
+            emit_top(take, k, slots, &s_cnt[3], emit);
+            found = k;
+        }
     }
     uint32_t p_out = 0;
     if (a.pos) p_out = *a.pos;
@@ -344,20 +453,23 @@ __global__ __launch_bounds__(kSpThreads) void sample_kernel(SampleArgs a) {
     __syncthreads();
 
     if (k <= 64) {
-        // One wave: bitonic sort in registers (descending), then softmax,
+        // One wave: each lane counts the keys above its own (all differ: the
+        // index is part of them) and puts it at that place, then softmax,
         // running sums, the top-p cut and the coin walk with lane scans.
         if (tid >= 64) return;
         const int lane = tid;
-        uint64_t v = (uint32_t)lane < k ? s_top[lane] : 0ull;
+        if ((uint32_t)lane >= found) s_top[lane] = 0;
+        // The wave's LDS accesses run in order; the fences keep the compiler's.
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        const uint64_t own = s_top[lane];
+        uint32_t rank = 0;
+        for (uint32_t i = 0; i < found; i += 4) {  // places past `found` hold 0
 #pragma unroll
-        for (int size = 2; size <= 64; size <<= 1) {
-#pragma unroll
-            for (int stride = size >> 1; stride > 0; stride >>= 1) {
-                const uint64_t o = __shfl_xor(v, stride);
-                const bool keep_max = ((lane & stride) == 0) == ((lane & size) == 0);
-                v = keep_max ? (v > o ? v : o) : (v < o ? v : o);
-            }
+            for (uint32_t u = 0; u < 4; ++u) rank += s_top[i + u] > own;
         }
+        if ((uint32_t)lane < found) s_sorted[rank] = own;
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        const uint64_t v = (uint32_t)lane < k ? s_sorted[lane] : 0ull;
         const bool in = (uint32_t)lane < k;
         const float x = sp_val((uint32_t)(v >> 32));
         const float xmax = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(x)));
