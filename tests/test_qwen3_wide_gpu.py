@@ -81,3 +81,44 @@ def test_wide_prefill_and_decode_vs_oracle(dev, weights_wide, graph, msl):
         assert toks[T + s + 1] == oracle.argmax(got), f"step {s} pick"
     assert m.position_host() == T + steps
     m.close()
+
+
+# One-token projections with the norm in front: the input requested ahead of
+# the weight rows or in trips with them, by grid size and row length (n = 1536,
+# 2560, 3584 and 4096 on either side of the lines: q/k/v of 1024, 4608, 6144 and
+# 8192 rows, gate/up of 1024 to 4096).
+@pytest.mark.parametrize("hidden,hq,hkv,F", [(1536, 4, 2, 1536), (1536, 32, 8, 4096),
+                                             (2560, 8, 4, 2048), (2560, 32, 16, 2560),
+                                             (3584, 28, 4, 1024), (4096, 8, 4, 1024)])
+def test_decode_projection_orders_vs_prefill(dev, hidden, hq, hkv, F):
+    """The logits of a decode step equal, within the oracle bars, those of a
+    prefill that ends with the same token (whose projections are GEMMs)."""
+    print(f"[step] decode projections hidden={hidden} {hq}/{hkv} F={F}", flush=True)
+    g = torch.Generator(device=dev).manual_seed(SEED)
+    V, T = 512, 24
+
+    def draw(*shape):
+        return (torch.randn(shape, generator=g, device=dev) * 0.02).to(torch.bfloat16)
+
+    ones = torch.ones(hidden, dtype=torch.bfloat16, device=dev)
+    layer = {"input_layernorm": ones, "q_proj": draw(hq * 128, hidden),
+             "k_proj": draw(hkv * 128, hidden), "v_proj": draw(hkv * 128, hidden),
+             "q_norm": ones[:128], "k_norm": ones[:128], "o_proj": draw(hidden, hq * 128),
+             "post_attention_layernorm": ones, "gate_proj": draw(F, hidden),
+             "up_proj": draw(F, hidden), "down_proj": draw(hidden, F)}
+    embed = draw(V, hidden)
+    ids = torch.randint(0, V, (T + 1,), generator=g, device=dev, dtype=torch.int32)
+    H.sync()
+    cfg = qwen3.make_config(num_layers=1, hidden_size=hidden, num_q_heads=hq, num_kv_heads=hkv,
+                            head_dim=128, intermediate_size=F, vocab_size=V, max_seq_len=64,
+                            max_prefill_tokens=32, rms_norm_eps=1e-6, rope_theta=1e6)
+    m = qwen3.Qwen3(cfg, {"embed_tokens": embed, "norm": ones, "lm_head": embed, "layers": [layer]})
+    m.prefill(ids, T)
+    pick = int(m.tokens_host(T + 1)[T])
+    m.decode(1, True)
+    got = m.logits_host()
+    ids[T] = pick
+    H.sync()
+    m.prefill(ids, T + 1)
+    check_logits(got, m.logits_host(), "decode vs prefill")
+    m.close()

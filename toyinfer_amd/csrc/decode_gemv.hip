@@ -201,16 +201,22 @@ __global__ __launch_bounds__(kDgThreads) void decode_gemv_kernel(DecodeGemvArgs 
 // block-cooperative kernel below; 16-wave workgroups on 32-48 CUs stream the
 // same matrices from HBM at under half the rate (8.5 us for 4 MB).  The
 // residual row is read at the start, by every lane (left to the compiler it is
-// read where it is added, another trip to memory at the end); the input goes
-// out ahead of the weights, whose flight then covers the norm; and the
-// arguments come in one round.  Those three: 0.675 -> 0.664 ms per Qwen3-0.6B
-// decode step.  The weight rows carry the non-temporal hint (read once per
-// step: 0.729 -> 0.666 ms together with the lm-head's).  Repeated from one
-// graph with weights from HBM, a launch takes 2.8 (o), 3.1 (down), 3.2 (q/k/v)
-// and 4.0 us (gate/up); with the weights in L2 2.2-3.1, an empty kernel 1.7.
+// read where it is added, another trip to memory at the end), and the
+// arguments come in one round: res 1536 x 1536 3.25 -> 3.0 us, 4096 x 2048 4.7
+// -> 4.5.  The weight rows carry the non-temporal hint (read once per step:
+// 0.729 -> 0.666 ms per Qwen3-0.6B decode step together with the lm-head's).
+// Repeated from one graph with weights from HBM, a launch takes 2.8 (o), 3.1
+// (down), 3.3 (q/k/v) and 4.1 us (gate/up); with the weights in L2 2.2-3.1, an
+// empty kernel 1.7.
+//
+// AHEAD (NORM only): all of the input and gamma is requested before the
+// weight rows, whose flight then covers the norm.  Every load of the wave is
+// then held in registers at once (170 of them for two 4096-wide rows, where
+// the rows in trips take 94), which pays while the grid's waves are resident
+// together: see dw_ahead_fits.
 constexpr int kDwWaves = 4;
 
-template <int RPW, int NCH, bool NORM, int EPI>
+template <int RPW, int NCH, bool NORM, int EPI, bool AHEAD>
 __global__ __launch_bounds__(64 * kDwWaves) void decode_gemv_wave_kernel(DecodeGemvArgs a) {
     constexpr int NR = EPI == kDgSwiglu ? 2 * RPW : RPW;
     if constexpr (EPI == kDgPlain)
@@ -249,14 +255,16 @@ __global__ __launch_bounds__(64 * kDwWaves) void decode_gemv_wave_kernel(DecodeG
     uint16_t res = 0;
     if constexpr (EPI == kDgResidual)
         res = __builtin_amdgcn_raw_buffer_load_b16(make_rsrc(seg_y + r0, 2 * nrows), 2 * lane, 0, 0);
-    // The input first: its sum of squares is taken while the rows arrive.
-#pragma unroll
-    for (int k = 0; k < NCH; ++k) {
+    auto load_input = [&](int k) __attribute__((always_inline)) {
         const uint32_t off = 16 * (lane + 64 * k);
         xv[k] = buf_load16(rx, off);
         if constexpr (NORM) gv[k] = buf_load16(make_rsrc(a.norm_w, row_bytes), off);
+    };
+    if constexpr (AHEAD) {
+#pragma unroll
+        for (int k = 0; k < NCH; ++k) load_input(k);
+        __builtin_amdgcn_sched_barrier(0);
     }
-    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int k = 0; k < NCH; ++k) {
         // Chunks past the row's end read zeros: their offset is moved past
@@ -266,8 +274,9 @@ __global__ __launch_bounds__(64 * kDwWaves) void decode_gemv_wave_kernel(DecodeG
 #pragma unroll
         for (int r = 0; r < NR; ++r)
             wv[r][k] = buf_load16_nt(rw[r / RPW], in ? (r % RPW) * row_bytes + off : 0x80000000u);
+        if constexpr (!AHEAD) load_input(k);
     }
-    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (AHEAD) __builtin_amdgcn_sched_barrier(0);
 
     if constexpr (NORM) {
         float ss = 0.0f;
@@ -315,8 +324,23 @@ __global__ __launch_bounds__(64 * kDwWaves) void decode_gemv_wave_kernel(DecodeG
         const float g = bf16_round(v), up = bf16_round(u);
         out = f32_to_bf16(up * (g * (1.0f / (1.0f + expf(-g)))));
     }
-    asm volatile("" : "+v"(out));  // computed (and the residual loaded) by every lane
+    // The residual form is computed, and so the residual loaded, by every lane
+    // (SwiGLU's exponential in every lane costs 1-3 % of gate/up).
+    if constexpr (EPI == kDgResidual) asm volatile("" : "+v"(out));
     if ((uint32_t)lane < nrows) seg_y[r0 + lane] = (uint16_t)out;
+}
+
+// Which grids run AHEAD: at most 12 row chunks per lane and 3072 waves (three
+// per SIMD; 2048 with gate and up).  Measured, us from a graph, weights from
+// HBM, in trips -> ahead: q/k/v of 2048 rows, n = 2560 6.3 -> 5.8, n = 4096 5.6
+// -> 5.35; 4096 rows, n = 2560 6.3 -> 5.8; 5120 rows 7.4 -> 7.1; beyond the
+// lines 8192 rows, n = 1536 5.8 -> 6.2, n = 2560 9.1 -> 9.3; 4096 rows, n = 4096
+// 7.4 -> 7.5; 16384 rows, n = 3584 19.5 -> 21.2; gate/up of 2048, n = 2560 5.85
+// -> 5.75, 2560 6.6 -> 7.1, 9728 17.2 -> 18.3, of 12288, n = 4096 31.6 -> 33.0.
+// Up to n = 1024 the two are level (0.05 us) and wide grids slower ahead (n =
+// 512, 16384 rows 4.65 -> 5.1).
+constexpr bool dw_ahead_fits(int rpw, int nch, int epi) {
+    return nch >= 4 && (epi == kDgSwiglu ? 2 : 1) * rpw * nch <= 12;
 }
 
 template <int RPW, int NCH, bool NORM, int EPI>
@@ -324,7 +348,11 @@ hipError_t dw_launch(const DecodeGemvArgs& a, hipStream_t stream) {
     uint32_t waves = 0;
     for (int s = 0; s < a.nseg; ++s) waves += (a.rows[s] + RPW - 1) / RPW;
     const uint32_t groups = (waves + kDwWaves - 1) / kDwWaves;
-    decode_gemv_wave_kernel<RPW, NCH, NORM, EPI><<<groups, 64 * kDwWaves, 0, stream>>>(a);
+    constexpr bool CAN = NORM && dw_ahead_fits(RPW, NCH, EPI);
+    if (CAN && waves <= (EPI == kDgSwiglu ? 2048u : 3072u))
+        decode_gemv_wave_kernel<RPW, NCH, NORM, EPI, CAN><<<groups, 64 * kDwWaves, 0, stream>>>(a);
+    else
+        decode_gemv_wave_kernel<RPW, NCH, NORM, EPI, false><<<groups, 64 * kDwWaves, 0, stream>>>(a);
     return hipGetLastError();
 }
 
