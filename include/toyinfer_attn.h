@@ -276,6 +276,16 @@ int toyinfer_gemm_segments_bf16(const void* hidden_states, uint32_t num_tokens, 
 int toyinfer_gemm_swiglu_bf16(const void* hidden_states, uint32_t num_tokens, uint32_t N,
                               const void* W_gate, const void* W_up, uint32_t M, void* out,
                               void* stream);
+/* The two calls above with the GEMM's tile chosen explicitly (extension, for
+ * tuning and tests): epilogue 0 = segments, 1 = segments with the residual
+ * add, 2 = SwiGLU (W and rows of gate and up, y[0] the output); tile 0 = by
+ * shape, as those calls do, 1..9 = 64x64, 96x64, 128x64, 128x128, 192x128,
+ * 256x128, 192x192, 256x192, 256x256 tokens x outputs.  The tile does not
+ * change a result bit.  TOYINFER_ERR_UNSUPPORTED for a tile at the few-token
+ * sizes that another kernel takes. */
+int toyinfer_gemm_tile_bf16(const void* hidden_states, uint32_t num_tokens, uint32_t N,
+                            uint32_t num_segments, const void* const* W, void* const* y,
+                            const uint32_t* rows, int epilogue, int tile, void* stream);
 
 /* ---- The rest of a Qwen3 decoder layer (for the model harness) ----
  * bf16 tensors need 4-byte alignment (16 bytes and sizes % 8 == 0 take the

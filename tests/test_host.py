@@ -77,6 +77,10 @@ def test_layer_op_validation():
     assert seg(P, 4, 256, 3, W, Y, R, 0, None) == UNSUPPORTED                 # GEMV-sized batch
     assert seg(P, 100, 96, 3, W, Y, R, 0, None) == UNSUPPORTED                # N % 64 != 0
     assert seg(P + 2, 100, 256, 3, W, Y, R, 0, None) == UNSUPPORTED           # unaligned input
+    tl = L.toyinfer_gemm_tile_bf16
+    assert tl(P, 1000, 256, 3, W, Y, R, 0, 10, None) == INVALID               # nine tile sizes
+    assert tl(P, 1000, 256, 3, W, Y, R, 3, 0, None) == INVALID                # three epilogues
+    assert tl(P, 1000, 256, 3, W, Y, R, 2, 1, None) == INVALID                # SwiGLU: gate and up
 
 
 def test_model_header_functions_exported_and_bound():

@@ -168,9 +168,8 @@ def test_batch_proj_shapes(dev, T, M, N):
     assert (got[T * M:] == SENTINEL).all()
 
 
-# The first two tile the chip with 256 x 256 tiles, with ragged tiles and
-# slice counts that are odd or tiny; 1371 x 6144 takes the 128 x 192 tiles
-# (its 128 x 128 grid would overflow the resident workgroups).
+# Full grids of the large tiles, with ragged tiles and slice counts that are
+# odd or tiny.
 @pytest.mark.parametrize("T,M,N", [(4096, 4096, 4096), (4000, 4100, 4160), (4096, 4096, 64),
                                    (2048, 4096, 4096), (1000, 1024, 4096), (512, 12288, 4096),
                                    (512, 4096, 12288), (1371, 6144, 1024)])
@@ -259,10 +258,11 @@ def test_gemm_residual_epilogue_equals_projection_then_add(dev, T, H, M):
 @pytest.mark.parametrize("T,hid,M", [(1371, 1024, 3072), (4096, 1024, 3072), (300, 512, 3072),
                                      (17, 256, 200), (33, 256, 204)])
 def test_gemm_swiglu_equals_projections_then_swiglu(dev, T, hid, M):
-    """Gate/up with SwiGLU in the GEMM epilogue (192 x 128, 256 x 256 and
-    128 x 128 tiles by grid size; a ragged last tile at M = 200; M = 204:
-    rows not 16-byte aligned) equals the two projections followed by
-    batch_swiglu_bf16x2, bit for bit."""
+    """Gate/up with SwiGLU in the epilogue equals the two projections followed
+    by batch_swiglu_bf16x2, bit for bit: the GEMM at sizes of the models, and
+    the few-token kernel (M = 200: a ragged last tile; M = 204: rows not
+    16-byte aligned).  Every GEMM tile size and its ragged tiles:
+    test_gemm_tile_sizes_and_epilogues."""
     print(f"[step] gemm swiglu T={T} hid={hid} M={M}", flush=True)
     g = torch.Generator(device=dev).manual_seed(39)
     x = torch.randn((T, hid), generator=g, device=dev).to(torch.bfloat16)
@@ -333,3 +333,46 @@ def test_few_token_segments_and_epilogues(dev, T, hid, rows):
             attn.batch_swiglu_bf16x2(ref, gu, exp, T, r)
             H.sync()
             assert torch.equal(out.view(torch.int16), exp.view(torch.int16)), f"swiglu, rows {r}"
+
+
+# Every tile size of the GEMM, at K of fewer slices than its ring has stages,
+# of as many and of one to three more, on ragged output tiles whose rows are
+# (520) and are not (204) whole 16-byte chunks, and on two token tiles of the
+# largest; 204 and 520 outputs leave 96- and 192-wide tiles and their halves
+# partial.
+GEMM_TILES = range(1, 10)
+
+
+@pytest.mark.parametrize("T,M,N", [(321, 204, 64), (321, 520, 128), (330, 204, 192), (513, 204, 256),
+                                   (400, 204, 320), (321, 520, 384), (321, 204, 448), (700, 520, 1024)])
+def test_gemm_tile_sizes_and_epilogues(dev, T, M, N):
+    print(f"[step] gemm tiles T={T} M={M} N={N}", flush=True)
+    g = torch.Generator(device=dev).manual_seed(42)
+    x = torch.randn((T, N), generator=g, device=dev).to(torch.bfloat16)
+    w, up = [(torch.randn((M, N), generator=g, device=dev) * 0.05).to(torch.bfloat16) for _ in range(2)]
+    old = torch.randn((T, M), generator=g, device=dev).to(torch.bfloat16)
+    # One rounding to bf16 and fp32 sums in any order.
+    ref = x.double() @ w.double().t()
+    slack = (x.double().abs() @ w.double().abs().t()) * 2.0 ** -20
+    first = None
+    for tile in GEMM_TILES:
+        print(f"  tile {tile}", flush=True)
+        bufs = [torch.full((T * M + 9,), SENTINEL_F, dtype=torch.bfloat16, device=dev) for _ in range(4)]
+        plain, also, res, glu = [b[:T * M].view(T, M) for b in bufs]
+        attn.gemm_tile_bf16(x, T, N, [w, up], [plain, also], [M, M], 0, tile)
+        res.copy_(old)
+        attn.gemm_tile_bf16(x, T, N, [w], [res], [M], 1, tile)
+        attn.gemm_tile_bf16(x, T, N, [w, up], [glu, None], [M, M], 2, tile)
+        H.sync()
+        assert all(bool((b[T * M:] == SENTINEL_F).all()) for b in bufs), f"tile {tile} wrote past the end"
+        if first is None:
+            err = (plain.double() - ref).abs()
+            assert bool((err <= ref.abs() * 2.0 ** -8 + slack).all()), f"max err {float(err.max())}"
+            added = (old.float() + plain.float()).to(torch.bfloat16)
+            exp = torch.empty_like(plain)
+            attn.batch_swiglu_bf16x2(plain, also, exp, T, M)
+            H.sync()
+            first = plain
+        assert torch.equal(plain.view(torch.int16), first.view(torch.int16)), f"tile {tile}"
+        assert torch.equal(res.view(torch.int16), added.view(torch.int16)), f"residual, tile {tile}"
+        assert torch.equal(glu.view(torch.int16), exp.view(torch.int16)), f"swiglu, tile {tile}"

@@ -64,6 +64,7 @@ SIGNATURES = {
     "toyinfer_batch_gemv_proj_bf16": (_i32, [_vp, _vp, _vp, _u32, _u32, _u32, _vp]),
     "toyinfer_gemm_segments_bf16": (_i32, [_vp, _u32, _u32, _u32, _vp, _vp, _vp, _i32, _vp]),
     "toyinfer_gemm_swiglu_bf16": (_i32, [_vp, _u32, _u32, _vp, _vp, _u32, _vp, _vp]),
+    "toyinfer_gemm_tile_bf16": (_i32, [_vp, _u32, _u32, _u32, _vp, _vp, _vp, _i32, _i32, _vp]),
     "toyinfer_rmsnorm_bf16": (_i32, [_vp, _vp, _vp, _vp, _f32, _u32, _vp]),
     "toyinfer_batch_rmsnorm_bf16": (_i32, [_vp, _vp, _vp, _vp, _f32, _u32, _u32, _vp]),
     "toyinfer_residual_add_bf16": (_i32, [_vp, _vp, _u32, _vp]),
@@ -381,6 +382,18 @@ def gemm_swiglu_bf16(hidden_states, num_tokens: int, N: int, W_gate, W_up, M: in
     _check("gemm_swiglu_bf16",
            LIB.toyinfer_gemm_swiglu_bf16(_ptr(hidden_states), num_tokens, N, _ptr(W_gate),
                                          _ptr(W_up), M, _ptr(out), _stream(stream)))
+
+
+def gemm_tile_bf16(hidden_states, num_tokens: int, N: int, Ws, ys, rows, epilogue: int, tile: int,
+                   stream=None) -> None:
+    """The two calls above (epilogue 0 segments, 1 with the residual add, 2
+    SwiGLU) at an explicit tile size, 1..9 (for tuning and tests)."""
+    _check("gemm_tile_bf16",
+           LIB.toyinfer_gemm_tile_bf16(_ptr(hidden_states), num_tokens, N, len(Ws),
+                                       (ctypes.c_void_p * len(Ws))(*[_ptr(w) for w in Ws]),
+                                       (ctypes.c_void_p * len(ys))(*[_ptr(y) for y in ys]),
+                                       (ctypes.c_uint32 * len(rows))(*rows), epilogue, tile,
+                                       _stream(stream)))
 
 
 # ------------------------------------------------- rest of a decoder layer

@@ -626,49 +626,48 @@ int toyinfer_batch_gemv_proj_bf16(const void* W, const void* hidden_states, void
                                            as_stream(stream)));
 }
 
-int toyinfer_gemm_segments_bf16(const void* hidden_states, uint32_t num_tokens, uint32_t N,
-                                uint32_t num_segments, const void* const* W, void* const* y,
-                                const uint32_t* rows, int residual, void* stream) {
-    if (!W || !y || !rows || num_segments == 0 || num_segments > 3 || N > kProjMaxN)
+int toyinfer_gemm_tile_bf16(const void* hidden_states, uint32_t num_tokens, uint32_t N,
+                            uint32_t num_segments, const void* const* W, void* const* y,
+                            const uint32_t* rows, int epilogue, int tile, void* stream) {
+    if (!W || !y || !rows || num_segments == 0 || num_segments > 3 || N > kProjMaxN ||
+        epilogue < 0 || epilogue > 2 || tile < 0 || tile > kGemmTiles)
+        return TOYINFER_ERR_INVALID_ARGUMENT;
+    if (epilogue == 2 && (num_segments != 2 || rows[0] != rows[1]))
         return TOYINFER_ERR_INVALID_ARGUMENT;
     GemmArgs g;
     g.x = static_cast<const uint16_t*>(hidden_states);
     g.T = num_tokens;
     g.N = N;
     g.nseg = (int)num_segments;
-    g.residual = residual != 0;
+    g.residual = epilogue == 1;
+    g.swiglu = epilogue == 2;
+    g.tile = tile;
     for (uint32_t s = 0; s < num_segments; ++s) {
-        const int st = proj_args(W[s], hidden_states, y[s], 2, num_tokens, rows[s], N);
+        void* out = y[epilogue == 2 ? 0 : s];
+        const int st = proj_args(W[s], hidden_states, out, 2, num_tokens, rows[s], N);
         if (st != TOYINFER_OK) return st;
         if (!proj_uses_gemm(num_tokens, N, W[s], hidden_states)) return TOYINFER_ERR_UNSUPPORTED;
+        if (tile && proj_uses_skinny(num_tokens, rows[s])) return TOYINFER_ERR_UNSUPPORTED;
         g.w[s] = static_cast<const uint16_t*>(W[s]);
-        g.y[s] = static_cast<uint16_t*>(y[s]);
+        if (epilogue != 2 || s == 0) g.y[s] = static_cast<uint16_t*>(out);
         g.rows[s] = rows[s];
     }
     return from_hip(launch_gemm(g, as_stream(stream)));
 }
 
+int toyinfer_gemm_segments_bf16(const void* hidden_states, uint32_t num_tokens, uint32_t N,
+                                uint32_t num_segments, const void* const* W, void* const* y,
+                                const uint32_t* rows, int residual, void* stream) {
+    return toyinfer_gemm_tile_bf16(hidden_states, num_tokens, N, num_segments, W, y, rows,
+                                   residual != 0, 0, stream);
+}
+
 int toyinfer_gemm_swiglu_bf16(const void* hidden_states, uint32_t num_tokens, uint32_t N,
                               const void* W_gate, const void* W_up, uint32_t M, void* out,
                               void* stream) {
-    if (N > kProjMaxN) return TOYINFER_ERR_INVALID_ARGUMENT;
-    for (const void* w : {W_gate, W_up}) {
-        const int st = proj_args(w, hidden_states, out, 2, num_tokens, M, N);
-        if (st != TOYINFER_OK) return st;
-        if (!proj_uses_gemm(num_tokens, N, w, hidden_states)) return TOYINFER_ERR_UNSUPPORTED;
-    }
-    GemmArgs g;
-    g.x = static_cast<const uint16_t*>(hidden_states);
-    g.T = num_tokens;
-    g.N = N;
-    g.nseg = 2;
-    g.w[0] = static_cast<const uint16_t*>(W_gate);
-    g.w[1] = static_cast<const uint16_t*>(W_up);
-    g.y[0] = static_cast<uint16_t*>(out);
-    g.rows[0] = M;
-    g.rows[1] = M;
-    g.swiglu = true;
-    return from_hip(launch_gemm(g, as_stream(stream)));
+    const void* const w[2] = {W_gate, W_up};
+    const uint32_t rows[2] = {M, M};
+    return toyinfer_gemm_tile_bf16(hidden_states, num_tokens, N, 2, w, &out, rows, 2, 0, stream);
 }
 
 static bool bf16_ok(const void* p) { return p && aligned(p, 4); }

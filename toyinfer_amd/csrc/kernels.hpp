@@ -202,7 +202,9 @@ struct GemmArgs {
     // SwiGLU epilogue: nseg = 2, w[0] gate and w[1] up (rows[0] == rows[1]),
     // y[0][t][m] = bf16(bf16(up) * silu(bf16(gate))).
     bool swiglu = false;
+    int tile = 0;  // 0: by shape; 1..kGemmTiles: the GEMM at that tile size, smallest first
 };
+constexpr int kGemmTiles = 9;
 hipError_t launch_gemm(const GemmArgs& g, hipStream_t stream);
 // The same for a few tokens, with K split over the waves of a workgroup
 // (another summation order).  launch_gemm sends each segment of `rows`

@@ -195,39 +195,41 @@ struct GmCfg {
 // slice is the time of a K slice while the rest of the chip idles (DMA and
 // operand reads for the small tiles, MFMAs for the large), load what a full
 // chip adds (shared caches, and the clock the power limit leaves).  Fitted
-// to 136 measured problems (T 20-4096, the q/k/v, o, gate/up + SwiGLU and
-// down projections of a 1024- and a 4096-wide layer): within 4-6 % rms of
-// every configuration's time, and the configuration it picks is on average
-// 0.3 % and at most 6 % slower than the fastest one.
+// to 830 measured problems with the weights in HBM (T 5-4096, the
+// projections of 512- to 5120-wide layers, outputs from 64 to 65536, N from
+// 64): within 11-19 % rms of every configuration's time, and the configuration
+// it picks is on average 0.5 % and at most 23 % slower than the fastest.  (A
+// fit to 136 problems of two layers, caches warm, took 64 x 64 tiles at N =
+// 128, T = 2000, 4096 outputs, 15.1 us, where 192 x 192 take 8.5.)
 struct GmCost {
     float fixed, round, slice, load;
 };
 struct GmMini : GmCfg<64, 64, 2, 2, 2, 4> {  // 4 waves of 32 x 32, two workgroups per CU
-    static constexpr GmCost COST{2.05f, 0.40f, 0.141f, 0.0425f};
+    static constexpr GmCost COST{2.33f, 0.53f, 0.223f, 0.060f};
 };
 struct GmSix : GmCfg<96, 64, 3, 2, 1, 4> {  // 6 waves of 32 x 32
-    static constexpr GmCost COST{1.2f, 1.9f, 0.175f, 0.076f};
+    static constexpr GmCost COST{1.45f, 1.62f, 0.240f, 0.082f};
 };
 struct GmFlat : GmCfg<128, 64, 4, 2, 1, 4> {  // 8 waves of 32 x 32
-    static constexpr GmCost COST{0.8f, 2.1f, 0.174f, 0.114f};
+    static constexpr GmCost COST{0.95f, 2.67f, 0.244f, 0.111f};
 };
 struct GmDeep : GmCfg<128, 128, 2, 4, 1, 4> {  // 8 waves of 64 x 32
-    static constexpr GmCost COST{0.6f, 3.4f, 0.260f, 0.185f};
+    static constexpr GmCost COST{0.71f, 2.85f, 0.352f, 0.225f};
 };
 struct GmTall : GmCfg<192, 128, 2, 4, 1, 3> {  // 8 waves of 96 x 32
-    static constexpr GmCost COST{0.0f, 5.9f, 0.322f, 0.279f};
+    static constexpr GmCost COST{0.33f, 3.48f, 0.473f, 0.277f};
 };
 struct GmHalf : GmCfg<256, 128, 4, 2, 1, 3> {  // 8 waves of 64 x 64
-    static constexpr GmCost COST{0.0f, 7.5f, 0.416f, 0.343f};
+    static constexpr GmCost COST{0.0f, 4.66f, 0.529f, 0.404f};
 };
 struct GmWide : GmCfg<192, 192, 2, 6, 1, 3> {  // 12 waves of 96 x 32
-    static constexpr GmCost COST{0.0f, 7.6f, 0.428f, 0.431f};
+    static constexpr GmCost COST{0.0f, 4.46f, 0.572f, 0.450f};
 };
 struct GmBroad : GmCfg<256, 192, 4, 2, 1, 2> {  // 8 waves of 64 x 96
-    static constexpr GmCost COST{0.0f, 7.0f, 0.713f, 0.434f};
+    static constexpr GmCost COST{0.28f, 4.60f, 0.849f, 0.583f};
 };
 struct GmLarge : GmCfg<256, 256, 2, 4, 1, 2> {  // 8 waves of 128 x 64
-    static constexpr GmCost COST{0.0f, 8.9f, 0.863f, 0.569f};
+    static constexpr GmCost COST{0.01f, 5.92f, 0.972f, 0.734f};
 };
 
 // LDS rows of BK bf16 (CPR 16-byte chunks); chunk c of row r sits at
@@ -395,7 +397,11 @@ __device__ __forceinline__ uint32_t gm_dma_offset(uint32_t blk, int lane, uint32
 // = 1371, 1024-wide layer: q/k/v 16.1 -> 14.5, o 10.8 -> 10.1, gate/up 25.3
 // -> 21.4, down 18.5 -> 15.4; T = 37: 6.1 -> 5.3, 9.2 -> 7.0, 12.6 -> 5.3,
 // 12.4 -> 8.9; T = 600, 4096-wide: 51 -> 32, 45 -> 26, 194 -> 120, 130 -> 74.
-template <typename C, bool SW>
+//
+// SHORT: at most ST slices, all requested at once and no ring (N = 64, T = 16,
+// 1024 outputs 3.06 -> 2.66 us, where ST - 1 requests past the end held up the
+// one slice).
+template <typename C, bool SW, bool SHORT>
 __global__ __launch_bounds__(C::THREADS, C::MINB) void gemm_kernel(GemmArgs g) {
     constexpr int IM = C::IM, JN = C::JN, BK = C::BK, KS = C::KS, ST = C::ST;
     const uint32_t T = g.T, N = g.N;
@@ -460,8 +466,7 @@ __global__ __launch_bounds__(C::THREADS, C::MINB) void gemm_kernel(GemmArgs g) {
     }
     // The next slice to load: its first column in A and in this wave's part
     // of B, and the bytes from there to the tile's end.  Past the last slice
-    // (the ring runs in whole rounds of ST) the ranges are empty: the loads
-    // give zeros, which add nothing.
+    // the ranges are empty: those loads give zeros, which nothing multiplies.
     const uint16_t* pa = x + (size_t)t0 * N;
     const uint16_t* pb = pick3(g.w, seg) + (size_t)m0 * N;
     if (SW && wave_s % 2) pb = g.w[1] + (size_t)m0 * N;
@@ -531,33 +536,61 @@ __global__ __launch_bounds__(C::THREADS, C::MINB) void gemm_kernel(GemmArgs g) {
         __builtin_amdgcn_sched_barrier(0);
         next_slice();
     };
-    dma_slice(s_0);
-    next_slice();
-    dma_slice(s_1);
-    next_slice();
-    if constexpr (ST > 2) {
-        dma_slice(s_2);
+    if constexpr (SHORT) {
+        uint16_t* const stage[4] = {s_0, s_1, s_2, s_3};
+#pragma unroll
+        for (int k = 0; k < ST; ++k)
+            if (k < (int)nk) {
+                dma_slice(stage[k]);
+                next_slice();
+            }
+        __builtin_amdgcn_s_waitcnt(kWaitVmLgkm0);
+        asm volatile("s_barrier" ::: "memory");
+#pragma unroll
+        for (int k = 0; k < ST; ++k)
+            if (k < (int)nk) {
+#pragma unroll
+                for (int s = 0; s < KS; ++s) {
+                    read(stage[k], s);
+                    mfmas(s);
+                }
+            }
+    } else {
+        dma_slice(s_0);
         next_slice();
-    }
-    if constexpr (ST > 3) {
-        dma_slice(s_3);
+        dma_slice(s_1);
         next_slice();
-    }
-    __builtin_amdgcn_s_waitcnt(wait_vmcnt_lgkm0((ST - 1) * DMAS));
-    asm volatile("s_barrier" ::: "memory");
-    read(s_0, 0);
-    for (uint32_t kt = 0; kt < nk; kt += ST) {
-        step(s_0, s_1);
-        if constexpr (ST == 2) {
-            step(s_1, s_0);
-        } else if constexpr (ST == 3) {
-            step(s_1, s_2);
-            step(s_2, s_0);
-        } else {
-            step(s_1, s_2);
-            step(s_2, s_3);
-            step(s_3, s_0);
+        if constexpr (ST > 2) {
+            dma_slice(s_2);
+            next_slice();
         }
+        if constexpr (ST > 3) {
+            dma_slice(s_3);
+            next_slice();
+        }
+        __builtin_amdgcn_s_waitcnt(wait_vmcnt_lgkm0((ST - 1) * DMAS));
+        asm volatile("s_barrier" ::: "memory");
+        read(s_0, 0);
+        // Whole rounds of the ring, then the nk % ST slices left (a further round
+        // would multiply zeros: at N = 1024 on three stages 18 slices' time for 16,
+        // at N = 128 on four stages 4 for 2).
+        uint32_t kt = 0;
+        for (; kt + ST <= nk; kt += ST) {
+            step(s_0, s_1);
+            if constexpr (ST == 2) {
+                step(s_1, s_0);
+            } else if constexpr (ST == 3) {
+                step(s_1, s_2);
+                step(s_2, s_0);
+            } else {
+                step(s_1, s_2);
+                step(s_2, s_3);
+                step(s_3, s_0);
+            }
+        }
+        if (kt < nk) step(s_0, s_1);
+        if (ST > 2 && kt + 1 < nk) step(s_1, s_2);
+        if (ST > 3 && kt + 2 < nk) step(s_2, s_3);
     }
     // The ring is free for the epilogue once every wave's last reads and
     // (empty) DMA are done.
@@ -673,7 +706,10 @@ uint32_t gemm_tiles(const GemmArgs& g) {
 
 template <typename C, bool SW = false>
 hipError_t gemm_launch(const GemmArgs& g, hipStream_t stream) {
-    gemm_kernel<C, SW><<<gemm_tiles<C, SW>(g), C::THREADS, 0, stream>>>(g);
+    if (g.N / kGmBK <= C::ST)
+        gemm_kernel<C, SW, true><<<gemm_tiles<C, SW>(g), C::THREADS, 0, stream>>>(g);
+    else
+        gemm_kernel<C, SW, false><<<gemm_tiles<C, SW>(g), C::THREADS, 0, stream>>>(g);
     return hipGetLastError();
 }
 
@@ -696,15 +732,17 @@ float gemm_cost(const GemmArgs& g, uint32_t cus) {
     return C::COST.fixed + rounds * (C::COST.round + slices * (C::COST.slice + C::COST.load * u));
 }
 
-// The configuration of least modelled cost.  Every one sums K in the same
-// MFMA order, so the choice does not change a result bit.
+// The configuration of least modelled cost, or the one that the caller names.
+// Every one sums K in the same MFMA order, so the choice does not change a
+// result bit.
 template <bool SW>
 hipError_t gemm_pick_launch(const GemmArgs& g, hipStream_t stream) {
     const uint32_t cus = (uint32_t)gemm_cus();
     hipError_t (*best)(const GemmArgs&, hipStream_t) = nullptr;
     float least = 0.0f;
+    int tile = 0;
     auto consider = [&](float cost, hipError_t (*launch)(const GemmArgs&, hipStream_t)) {
-        if (best == nullptr || cost < least) {
+        if (g.tile ? ++tile == g.tile : best == nullptr || cost < least) {
             least = cost;
             best = launch;
         }
@@ -752,6 +790,8 @@ hipError_t launch_batch_proj_bf16(const uint16_t* W, const uint16_t* x, uint16_t
 }
 
 hipError_t launch_gemm(const GemmArgs& g, hipStream_t stream) {
+    if (g.tile)
+        return g.swiglu ? gemm_pick_launch<true>(g, stream) : gemm_pick_launch<false>(g, stream);
     if (g.swiglu)
         return proj_uses_skinny(g.T, g.rows[0]) ? launch_gemm_skinny(g, stream)
                                                 : gemm_pick_launch<true>(g, stream);
