@@ -281,8 +281,9 @@ int toyinfer_gemm_swiglu_bf16(const void* hidden_states, uint32_t num_tokens, ui
  * add, 2 = SwiGLU (W and rows of gate and up, y[0] the output); tile 0 = by
  * shape, as those calls do, 1..9 = 64x64, 96x64, 128x64, 128x128, 192x128,
  * 256x128, 192x192, 256x192, 256x256 tokens x outputs.  The tile does not
- * change a result bit.  TOYINFER_ERR_UNSUPPORTED for a tile at the few-token
- * sizes that another kernel takes. */
+ * change a result bit.  TOYINFER_ERR_UNSUPPORTED, where a segment is of the
+ * few-token sizes that another kernel may take, for the tiles that do not sum
+ * in its order: 5..9, and all with SwiGLU. */
 int toyinfer_gemm_tile_bf16(const void* hidden_states, uint32_t num_tokens, uint32_t N,
                             uint32_t num_segments, const void* const* W, void* const* y,
                             const uint32_t* rows, int epilogue, int tile, void* stream);

@@ -11,6 +11,8 @@ element loads; 1, 2, 4 and 8 rows per workgroup; the MFMA GEMM with ragged
 token and output tiles) and check that nothing past num_tokens * M is
 written.  At full projection sizes the check is a torch fp32 product.
 """
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -376,3 +378,53 @@ def test_gemm_tile_sizes_and_epilogues(dev, T, M, N):
         assert torch.equal(plain.view(torch.int16), first.view(torch.int16)), f"tile {tile}"
         assert torch.equal(res.view(torch.int16), added.view(torch.int16)), f"residual, tile {tile}"
         assert torch.equal(glu.view(torch.int16), exp.view(torch.int16)), f"swiglu, tile {tile}"
+
+
+def graph_nodes(fn):
+    """Kernels that fn launches on the current stream."""
+    stream = torch.cuda.Stream()
+    with torch.cuda.stream(stream):
+        fn()
+    H.sync()
+    graph = torch.cuda.CUDAGraph(keep_graph=True)
+    with torch.cuda.graph(graph, stream=stream):
+        fn()
+    n = ctypes.c_size_t(0)
+    status = attn.LIB.hipGraphGetNodes(ctypes.c_void_p(graph.raw_cuda_graph()), None, ctypes.byref(n))
+    assert status == 0
+    return n.value
+
+
+# Stacks around the few-token line, some segments of which are summed in the
+# few-token kernel's order: q/k/v of 1024-, 2560- and 4096-wide layers, K of
+# fewer than eight, of eight and of one more slices, ragged rows that are not
+# whole 16-byte chunks, and stacks that are all of one order.
+@pytest.mark.parametrize("T,hid,rows", [
+    (160, 1024, (2048, 1024, 1024)), (200, 1024, (2048, 1024, 1024)), (320, 1024, (1024, 1024)),
+    (64, 2560, (4096, 1024, 1024)), (128, 4096, (4096, 1024, 1024)), (97, 320, (3072, 130, 33)),
+    (81, 512, (4096, 204, 4095)), (161, 576, (2049, 17, 300)), (5, 1024, (8193, 8, 16)),
+    (33, 1024, (2048, 1024, 1024)), (200, 256, (2048, 1024, 1024)), (5, 320, (1, 1, 1))])
+def test_stacks_around_the_few_token_line(dev, T, hid, rows):
+    """A stack is one launch and each segment's bits are those of the
+    projection by itself (and with the residual, of the add after it), at
+    every tile size that takes it."""
+    print(f"[step] stack T={T} hid={hid} rows={rows}", flush=True)
+    g = torch.Generator(device=dev).manual_seed(43)
+    x = torch.randn((T, hid), generator=g, device=dev).to(torch.bfloat16)
+    ws = [(torch.randn((r, hid), generator=g, device=dev) * 0.05).to(torch.bfloat16) for r in rows]
+    old = [torch.randn((T, r), generator=g, device=dev).to(torch.bfloat16) for r in rows]
+    ref = [torch.empty_like(o) for o in old]
+    for w, y, r in zip(ws, ref, rows):
+        attn.batch_gemv_proj_bf16(w, x, y, T, r, hid)
+    added = [(o.float() + y.float()).to(torch.bfloat16) for o, y in zip(old, ref)]
+    for tile in range(5):
+        print(f"  tile {tile}", flush=True)
+        ys, res = [torch.full_like(o, SENTINEL_F) for o in old], [o.clone() for o in old]
+        attn.gemm_tile_bf16(x, T, hid, ws, ys, rows, 0, tile)
+        attn.gemm_tile_bf16(x, T, hid, ws, res, rows, 1, tile)
+        H.sync()
+        for y, s, e, a, r in zip(ys, res, ref, added, rows):
+            assert torch.equal(y.view(torch.int16), e.view(torch.int16)), f"tile {tile}, rows {r}"
+            assert torch.equal(s.view(torch.int16), a.view(torch.int16)), f"residual, tile {tile}, rows {r}"
+    out = [torch.empty_like(o) for o in old]
+    assert graph_nodes(lambda: attn.gemm_segments_bf16(x, T, hid, ws, out, rows)) == 1

@@ -647,7 +647,8 @@ int toyinfer_gemm_tile_bf16(const void* hidden_states, uint32_t num_tokens, uint
         const int st = proj_args(W[s], hidden_states, out, 2, num_tokens, rows[s], N);
         if (st != TOYINFER_OK) return st;
         if (!proj_uses_gemm(num_tokens, N, W[s], hidden_states)) return TOYINFER_ERR_UNSUPPORTED;
-        if (tile && proj_uses_skinny(num_tokens, rows[s])) return TOYINFER_ERR_UNSUPPORTED;
+        if ((epilogue == 2 ? tile : tile > 4) && proj_uses_skinny(num_tokens, rows[s], N))
+            return TOYINFER_ERR_UNSUPPORTED;
         g.w[s] = static_cast<const uint16_t*>(W[s]);
         if (epilogue != 2 || s == 0) g.y[s] = static_cast<uint16_t*>(out);
         g.rows[s] = rows[s];

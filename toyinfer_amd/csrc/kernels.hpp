@@ -207,18 +207,34 @@ struct GemmArgs {
 constexpr int kGemmTiles = 9;
 hipError_t launch_gemm(const GemmArgs& g, hipStream_t stream);
 // The same for a few tokens, with K split over the waves of a workgroup
-// (another summation order).  launch_gemm sends each segment of `rows`
-// outputs there by T and rows alone, so that a stacked segment, a gate/up
-// pair and the projection by itself give the same bits.  The line: the ring
-// GEMM's 64 x 64 tiles fill the CUs from about T rows = 2^20 on, and each of
-// its tiles reads a quarter of the bytes per output (measured, weights from
-// HBM, ring -> K split, us: M = 1024, N = 3072, T = 256 16.9 -> 9.4; M = 2560,
-// N = 4096, T = 128 20.9 -> 13.1, T = 256 20.8 -> 20.6; M = 4096, N = 4096, T =
-// 64 21.6 -> 13.5, T = 100 19.7 -> 18.9, T = 192 21.3 -> 23.2; gate/up of 9728,
-// N = 2560, T = 37 29.7 -> 34.2).
-inline bool proj_uses_skinny(uint32_t T, uint32_t rows) {
-    return T <= 320 && (uint64_t)T * rows <= 5u << 16;
+// (another summation order).  Which order an element is summed in follows from
+// T, N and its segment's rows alone, so that a stacked segment, a gate/up pair
+// and the projection by itself give the same bits; launch_gemm chooses the
+// kernel for the whole call, a stack in one launch (proj.hip's kGmMixed sums
+// either order).
+//
+// The line: one block of 32 outputs x 48 tokens per CU, one round (a constant:
+// the bits do not depend on the device), which reads each weight once or a few
+// times and waits for N / 512 chunks in turn, where the GEMM's tiles wait for
+// N / 64.  With more blocks the GEMM's 64 x 64 tiles, each a quarter of the
+// reads per output, are faster: weights from HBM, K split / GEMM, us: N = 2048,
+// rows 1024, T = 320 8.8 / 12.0; N = 1024, rows 2048, T = 161 6.1 / 7.6, T = 200
+// (320 blocks) 9.2 / 7.4; rows 4096, T = 96 6.8 / 7.8, T = 128 (384 blocks) 10.1 /
+// 8.2; rows 20480, T = 16 (640) 15.2 / 12.2; N = 2560, rows 10240, T = 24 (320) 19.5
+// / 16.1; N = 4096 is level beyond the line (rows 3072, T = 97 18.3 /
+// 19.6; rows 20480, T = 8 38.8 / 40.6; gate/up of 12288 40.6 / 42.7), and T rows
+// <= 327680 is the line there.  Up to N = 256 few waves have a chunk of their
+// own and the GEMM asks for all of K at once (N = 64, rows 1024, T = 16 3.05 /
+// 2.66).
+constexpr uint32_t kSkinnyRound = 256;
+__host__ __device__ inline uint64_t skinny_tiles(uint32_t T, uint32_t rows) {
+    return (uint64_t)((rows + 31) / 32) * ((T + 47) / 48);
 }
+__host__ __device__ inline bool proj_uses_skinny(uint32_t T, uint32_t rows, uint32_t N) {
+    return T <= 320 && N > 256 && (uint64_t)T * rows <= 5u << 16 &&
+           (N >= 4096 || skinny_tiles(T, rows) <= kSkinnyRound);
+}
+int gemm_cus();  // compute units of the device
 hipError_t launch_gemm_skinny(const GemmArgs& g, hipStream_t stream);
 
 // ------------------------------------------------- fused decode projections

@@ -14,8 +14,9 @@
 //    token, so the tails need no branches.  The weight rows, read once per
 //    call, carry the non-temporal hint (the lm-head's 1.24 GB then streams
 //    at 6.95 TB/s where plain loads reach 6.2).
-//  * gemm_kernel: MFMA-bound (prefill, T > kGemvMaxTokens).  K in 64-wide
-//    slices through a ring of two to four LDS stages by buffer-load DMA,
+//  * gemm_kernel: MFMA-bound (prefill, T > kGemvMaxTokens, but for the small
+//    products of a few tokens, which proj_skinny.hip has).  K in 64-wide slices
+//    through a ring of two to four LDS stages by buffer-load DMA,
 //    v_mfma_f32_32x32x16_bf16 on 32 x 32 blocks.  Nine tile sizes from 64 x 64
 //    to 256 x 256, picked by a cost model of tiles, rounds and slices.  Tiles
 //    are ordered in 8 x 8 groups and the groups are dealt to XCDs in
@@ -23,6 +24,7 @@
 //    in that XCD's L2.  The results leave through LDS as whole 16-byte chunks
 //    of token rows.
 #include <cmath>
+#include <type_traits>
 
 #include "common.hpp"
 #include "kernels.hpp"
@@ -172,15 +174,15 @@ constexpr int kGmBK = 64;    // K granularity every GEMM configuration handles
 constexpr int kGmGroup = 8;  // tile groups of 8 x 8
 
 // Block tile BM (tokens) x BN (outputs) on a WGM x WGN grid of waves; each
-// wave owns IM x JN blocks of 32 x 32.  K advances in slices of kGmBK (KS
-// k-steps of 16) through a ring of ST LDS stages.
+// wave owns IM x JN blocks of 32 x 32.  K advances in slices of kGmBK
+// through a ring of ST LDS stages.
 template <int BM_, int BN_, int WGM_, int WGN_, int MINB_, int ST_>
 struct GmCfg {
     static constexpr int BM = BM_, BN = BN_, WGM = WGM_, WGN = WGN_, MINB = MINB_, ST = ST_;
     static constexpr int BK = kGmBK;
     static constexpr int WAVES = WGM * WGN, THREADS = 64 * WAVES;
     static constexpr int IM = BM / WGM / 32, JN = BN / WGN / 32;
-    static constexpr int KS = BK / 16, CPR = BK / 8, RPB = 64 / CPR;  // chunks per row, rows per DMA
+    static constexpr int RPB = 8;  // rows per DMA instruction
     static constexpr int A_ELEMS = BM * BK, B_ELEMS = BN * BK;
     static constexpr int A_BLOCKS = BM / RPB;                  // DMA instructions per slice of A
     static constexpr int BLOCKS = (BM + BN) / RPB;             // and in all
@@ -232,21 +234,14 @@ struct GmLarge : GmCfg<256, 256, 2, 4, 1, 2> {  // 8 waves of 128 x 64
     static constexpr GmCost COST{0.01f, 5.92f, 0.972f, 0.734f};
 };
 
-// LDS rows of BK bf16 (CPR 16-byte chunks); chunk c of row r sits at
-// c ^ gm_swz<CPR>(r).  A 16-byte LDS read serves 16 lanes per cycle from
-// 64 banks (256 bytes), and the MFMA operand reads put 16 consecutive rows
-// on 16 consecutive lanes, all at one logical chunk: with 256-byte rows
-// (CPR 16) the swizzle r & 15 gives the 16 rows 16 different chunks; with
-// 128-byte rows (CPR 8) rows r and r + 1 share a 256-byte bank line (r & 1
-// picks its half), so the 8 rows of each parity need different chunks:
-// (r >> 1) & 7.  (A swizzle r & 7 had rows r and r + 8 meet on the same
-// banks: 4 conflict cycles per read.)  One DMA instruction fills 64 / CPR
-// rows: lane l loads row l / CPR, physical chunk l % CPR, i.e. logical
-// chunk (l % CPR) ^ gm_swz<CPR>(row).
-template <int CPR>
-__device__ __forceinline__ uint32_t gm_swz(uint32_t row) {
-    return CPR == 16 ? row & 15 : (row >> 1) & 7;
-}
+// LDS rows of BK bf16 (128 bytes, eight 16-byte chunks); chunk c of row r
+// sits at c ^ gm_swz(r).  A 16-byte LDS read serves 16 lanes per cycle from 64
+// banks (256 bytes), and the MFMA operand reads put 16 consecutive rows on 16
+// consecutive lanes, all at one logical chunk: rows r and r + 1 share a
+// 256-byte bank line (r & 1 picks its half), so the 8 rows of each parity need
+// different chunks.  (A swizzle r & 7 had rows r and r + 8 meet on the same
+// banks: 4 conflict cycles per read.)
+__device__ __forceinline__ uint32_t gm_swz(uint32_t row) { return (row >> 1) & 7; }
 
 struct GmTile {
     uint32_t tt, tm;  // token tile, output tile
@@ -366,18 +361,17 @@ __device__ __forceinline__ uint4 add_bf16x8(uint4 a, uint4 b) {
     return make_uint4(o[0], o[1], o[2], o[3]);
 }
 
-// DMA instruction `blk` of a slice fills the 64 / CPR tile rows from
-// (64 / CPR) blk on (the A rows, then the B rows) of the stage at st; lane l
-// loads row l / CPR's physical chunk l % CPR, i.e. logical chunk (l % CPR) ^
-// gm_swz<CPR>(row).  SW: 16 gate and 16 up rows make a 32-row block of B,
+// DMA instruction `blk` of a slice fills the eight tile rows from 8 blk on
+// (the A rows, then the B rows) of the stage at st; lane l loads row l / 8's
+// physical chunk l % 8, i.e. logical chunk (l % 8) ^ gm_swz(row).  SW: 16 gate and 16 up rows make a 32-row block of B,
 // positions p with bit 3 clear gate, the others up, both of the 16 output
 // columns 8 (p / 16) + p % 8, so that a lane's accumulator values 8 q + u
 // and 8 q + 4 + u (u < 4) are gate and up of one output; the eight rows of
 // a DMA instruction are all of one kind.
 template <typename C, bool SW>
 __device__ __forceinline__ uint32_t gm_dma_offset(uint32_t blk, int lane, uint32_t row_bytes) {
-    const uint32_t r = C::RPB * blk + lane / C::CPR;  // tile row
-    const uint32_t logical = (lane % C::CPR) ^ gm_swz<C::CPR>(r);
+    const uint32_t r = C::RPB * blk + lane / 8;  // tile row
+    const uint32_t logical = (lane % 8) ^ gm_swz(r);
     uint32_t src = r < (uint32_t)C::BM ? r : r - C::BM;
     if (SW && r >= (uint32_t)C::BM)
         src = 16 * (src / 32) + 8 * (src / 16 % 2) + src % 8;
@@ -398,12 +392,25 @@ __device__ __forceinline__ uint32_t gm_dma_offset(uint32_t blk, int lane, uint32
 // -> 21.4, down 18.5 -> 15.4; T = 37: 6.1 -> 5.3, 9.2 -> 7.0, 12.6 -> 5.3,
 // 12.4 -> 8.9; T = 600, 4096-wide: 51 -> 32, 45 -> 26, 194 -> 120, 130 -> 74.
 //
-// SHORT: at most ST slices, all requested at once and no ring (N = 64, T = 16,
-// 1024 outputs 3.06 -> 2.66 us, where ST - 1 requests past the end held up the
-// one slice).
-template <typename C, bool SW, bool SHORT>
+// kGmShort: at most ST slices, all requested at once and no ring (N = 64, T =
+// 16, 1024 outputs 3.06 -> 2.66 us, where ST - 1 requests past the end held up
+// the one slice).
+//
+// kGmMixed: a stack of which some segments are summed as the few-token kernel
+// sums them (proj_uses_skinny), so that each element has the bits it has by
+// itself: the slices in that kernel's order (every eighth, from slice 0, then
+// from slice 1, ...), its MFMA, and eight partials added one after another.
+// One launch of every segment's tiles, where the two kernels in turn cost a
+// launch and left CUs idle twice.  Weights from HBM, us, two launches -> one (the
+// GEMM of before the few-token kernel): q/k/v of a 1024-wide layer, T = 160 10.8
+// -> 8.0 (10.0), T = 320 18.9 -> 9.6 (10.4); 2560-wide, T = 96 23.7 -> 15.3 (20.7),
+// T = 256 33.0 -> 22.9 (21.4, on slices of 128); 4096-wide, T = 128 33.1 -> 22.8
+// (31.0).  Every segment in the GEMM's own order takes 0.2 us less.
+enum GmForm : int { kGmRing, kGmShort, kGmMixed };
+
+template <typename C, bool SW, int FORM>
 __global__ __launch_bounds__(C::THREADS, C::MINB) void gemm_kernel(GemmArgs g) {
-    constexpr int IM = C::IM, JN = C::JN, BK = C::BK, KS = C::KS, ST = C::ST;
+    constexpr int IM = C::IM, JN = C::JN, BK = C::BK, ST = C::ST;
     const uint32_t T = g.T, N = g.N;
     const uint16_t* __restrict__ x = g.x;
     // One array per stage (A rows, then B rows), so that the compiler can
@@ -433,15 +440,8 @@ __global__ __launch_bounds__(C::THREADS, C::MINB) void gemm_kernel(GemmArgs g) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int wr = wave / C::WGN, wc = wave % C::WGN;
 
-    // Operand read offsets (elements) inside a stage for block 0, per
-    // k-step; block i adds 32 i rows.
-    int a_off[KS], b_off[KS];
-#pragma unroll
-    for (int s = 0; s < KS; ++s) {
-        const int chunk = (2 * s + (lane >> 5)) ^ gm_swz<C::CPR>(lane & 31);  // rows differ by 32 i
-        a_off[s] = (32 * IM * wr + (lane & 31)) * BK + 8 * chunk;
-        b_off[s] = C::A_ELEMS + (32 * JN * wc + (lane & 31)) * BK + 8 * chunk;
-    }
+    // Whether this tile's segment is summed in the few-token kernel's order.
+    const bool split = FORM == kGmMixed && proj_uses_skinny(T, M, N);
 
     f32x16_t acc[IM][JN];
 #pragma unroll
@@ -480,118 +480,179 @@ __global__ __launch_bounds__(C::THREADS, C::MINB) void gemm_kernel(GemmArgs g) {
         for (int j = 0; j < C::DMAS; ++j)
             dma16(C::WAVES * j < C::A_BLOCKS ? ra : rb, st + 512 * d_blk[j], d_off[j]);
     };
-    auto next_slice = [&]() __attribute__((always_inline)) {
-        pa += BK;
-        pb += BK;
-        a_left -= 2 * BK;
-        b_left -= 2 * BK;
-        k_left -= k_left != 0;
+    auto advance = [&](int slices) __attribute__((always_inline)) {  // or back
+        pa += slices * BK;
+        pb += slices * BK;
+        a_left -= (uint32_t)(2 * BK * slices);
+        b_left -= (uint32_t)(2 * BK * slices);
     };
-    // Operands of k-step s + 1 are read while the MFMAs of k-step s run (two
-    // register sets; KS is even, so a slice starts on set 0).
-    bf16x8_t a[2][IM], b[2][JN];
-    auto read = [&](const uint16_t* st, int s) __attribute__((always_inline)) {
+    // The products of this tile, in blocks of BLK x BLK: k-steps of 512 / BLK,
+    // whose operands lane l reads as row l % BLK, k 8 (l / BLK).
+    auto products = [&](auto split_order) __attribute__((always_inline)) {
+        constexpr bool SPLIT = decltype(split_order)::value;
+        constexpr int BLK = SPLIT ? 16 : 32;
+        constexpr int STEPS = BK * BLK / 512, AM = 32 / BLK * IM, BN = 32 / BLK * JN;
+        // Operand read offsets (elements) inside a stage for block 0, per
+        // k-step; block i adds BLK i rows, which the swizzle does not see.
+        int a_off[STEPS], b_off[STEPS];
 #pragma unroll
-        for (int i = 0; i < IM; ++i)
-            a[s & 1][i] = as_bf16x8(*reinterpret_cast<const uint4*>(st + a_off[s] + 32 * BK * i));
-#pragma unroll
-        for (int j = 0; j < JN; ++j)
-            b[s & 1][j] = as_bf16x8(*reinterpret_cast<const uint4*>(st + b_off[s] + 32 * BK * j));
-    };
-    auto mfmas = [&](int s) __attribute__((always_inline)) {
-#pragma unroll
-        for (int i = 0; i < IM; ++i)
-#pragma unroll
-            for (int j = 0; j < JN; ++j)
-                acc[i][j] = mfma32x32x16(b[s & 1][j], a[s & 1][i], acc[i][j]);  // W rows first
-    };
-    // Slice kt, in `cur`, its first operands already in registers: the MFMAs
-    // of k-steps 0 .. KS - 2; then, with the last k-step's operands in
-    // registers too, the hand-over (this wave's reads of cur and its part of
-    // slice kt + 1 have landed, then every wave's have), the first operand
-    // reads of slice kt + 1 and the DMA of slice kt + ST into cur, all spread
-    // over the MFMAs of the last k-step.
-    constexpr int DMAS = C::DMAS;
-    auto step = [&](uint16_t* cur, const uint16_t* nxt) __attribute__((always_inline)) {
-#pragma unroll
-        for (int s = 0; s < KS - 1; ++s) {
-            read(cur, s + 1);
-            mfmas(s);
-            __builtin_amdgcn_sched_group_barrier(0x100, IM + JN, 0);
-            __builtin_amdgcn_sched_group_barrier(0x008, IM * JN, 0);
+        for (int s = 0; s < STEPS; ++s) {
+            const int row = lane % BLK, chunk = (64 / BLK * s + lane / BLK) ^ gm_swz(row);
+            a_off[s] = (32 * IM * wr + row) * BK + 8 * chunk;
+            b_off[s] = C::A_ELEMS + (32 * JN * wc + row) * BK + 8 * chunk;
         }
-        __builtin_amdgcn_sched_barrier(0);
-        __builtin_amdgcn_s_waitcnt(wait_vmcnt_lgkm0((ST - 2) * DMAS));
-        asm volatile("s_barrier" ::: "memory");
-        __builtin_amdgcn_sched_barrier(0);
-        read(nxt, 0);
-        dma_slice(cur);
-        mfmas(KS - 1);
-        __builtin_amdgcn_sched_group_barrier(0x100, IM + JN, 0);
+        f32x4_t part[AM][BN];
+        if constexpr (SPLIT) {
 #pragma unroll
-        for (int k = 0; k < IM * JN; ++k) {
-            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-            __builtin_amdgcn_sched_group_barrier(0x020, (DMAS + IM * JN - 1) / (IM * JN), 0);
+            for (int i = 0; i < AM; ++i)
+#pragma unroll
+                for (int j = 0; j < BN; ++j) part[i][j] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
         }
-        __builtin_amdgcn_sched_barrier(0);
-        next_slice();
-    };
-    if constexpr (SHORT) {
-        uint16_t* const stage[4] = {s_0, s_1, s_2, s_3};
+        // Operands of k-step s + 1 are read while the MFMAs of k-step s run
+        // (two register sets; STEPS is even, so a slice starts on set 0).
+        bf16x8_t a[2][AM], b[2][BN];
+        auto read = [&](const uint16_t* st, int s) __attribute__((always_inline)) {
 #pragma unroll
-        for (int k = 0; k < ST; ++k)
-            if (k < (int)nk) {
-                dma_slice(stage[k]);
+            for (int i = 0; i < AM; ++i)
+                a[s & 1][i] = as_bf16x8(*reinterpret_cast<const uint4*>(st + a_off[s] + BLK * BK * i));
+#pragma unroll
+            for (int j = 0; j < BN; ++j)
+                b[s & 1][j] = as_bf16x8(*reinterpret_cast<const uint4*>(st + b_off[s] + BLK * BK * j));
+        };
+        auto mfmas = [&](int s) __attribute__((always_inline)) {
+#pragma unroll
+            for (int i = 0; i < AM; ++i)
+#pragma unroll
+                for (int j = 0; j < BN; ++j) {  // W rows first
+                    if constexpr (SPLIT)
+                        part[i][j] = mfma16x16x32(b[s & 1][j], a[s & 1][i], part[i][j]);
+                    else
+                        acc[i][j] = mfma32x32x16(b[s & 1][j], a[s & 1][i], acc[i][j]);
+                }
+        };
+        // SPLIT: the next slice is eight on, or the first of the next partial.
+        uint32_t slice = 0, partial = 0, partial_left = (nk + 7) / 8;
+        auto next_slice = [&]() __attribute__((always_inline)) {
+            if constexpr (SPLIT) {
+                const uint32_t to = slice + 8 < nk ? slice + 8 : slice % 8 + 1;
+                advance((int)to - (int)slice);
+                slice = to;
+            } else {
+                advance(1);
+            }
+            k_left -= k_left != 0;
+        };
+        // SPLIT: a finished partial is added to the sums (the 16 x 16 blocks
+        // of a 32 x 32 one at values 4 (2 J + I) on, J its half of the outputs, I
+        // of the tokens).
+        auto slice_done = [&]() __attribute__((always_inline)) {
+            if constexpr (SPLIT) {
+                if (--partial_left != 0) return;
+                partial_left = (nk - ++partial + 7) / 8;
+#pragma unroll
+                for (int i = 0; i < AM; ++i)
+#pragma unroll
+                    for (int j = 0; j < BN; ++j)
+#pragma unroll
+                        for (int v = 0; v < 4; ++v) {
+                            acc[i / 2][j / 2][4 * (2 * (j % 2) + i % 2) + v] += part[i][j][v];
+                            part[i][j][v] = 0.0f;
+                        }
+            }
+        };
+        if constexpr (FORM == kGmShort) {
+            uint16_t* const stage[4] = {s_0, s_1, s_2, s_3};
+#pragma unroll
+            for (int k = 0; k < ST; ++k)
+                if (k < (int)nk) {
+                    dma_slice(stage[k]);
+                    next_slice();
+                }
+            __builtin_amdgcn_s_waitcnt(kWaitVmLgkm0);
+            asm volatile("s_barrier" ::: "memory");
+#pragma unroll
+            for (int k = 0; k < ST; ++k)
+                if (k < (int)nk) {
+#pragma unroll
+                    for (int s = 0; s < STEPS; ++s) {
+                        read(stage[k], s);
+                        mfmas(s);
+                    }
+                }
+        } else {
+            // Slice kt, in `cur`, its first operands already in registers: the
+            // MFMAs of all k-steps but the last; then, with the last k-step's
+            // operands in registers too, the hand-over (this wave's reads of cur
+            // and its part of slice kt + 1 have landed, then every wave's have),
+            // the first operand reads of slice kt + 1 and the DMA of slice kt +
+            // ST into cur, all spread over the MFMAs of the last k-step.
+            constexpr int DMAS = C::DMAS;
+            auto step = [&](uint16_t* cur, const uint16_t* nxt) __attribute__((always_inline)) {
+#pragma unroll
+                for (int s = 0; s < STEPS - 1; ++s) {
+                    read(cur, s + 1);
+                    mfmas(s);
+                    __builtin_amdgcn_sched_group_barrier(0x100, AM + BN, 0);
+                    __builtin_amdgcn_sched_group_barrier(0x008, AM * BN, 0);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+                __builtin_amdgcn_s_waitcnt(wait_vmcnt_lgkm0((ST - 2) * DMAS));
+                asm volatile("s_barrier" ::: "memory");
+                __builtin_amdgcn_sched_barrier(0);
+                read(nxt, 0);
+                dma_slice(cur);
+                mfmas(STEPS - 1);
+                __builtin_amdgcn_sched_group_barrier(0x100, AM + BN, 0);
+#pragma unroll
+                for (int k = 0; k < AM * BN; ++k) {
+                    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                    __builtin_amdgcn_sched_group_barrier(0x020, (DMAS + AM * BN - 1) / (AM * BN), 0);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+                next_slice();
+                slice_done();
+            };
+            dma_slice(s_0);
+            next_slice();
+            dma_slice(s_1);
+            next_slice();
+            if constexpr (ST > 2) {
+                dma_slice(s_2);
                 next_slice();
             }
-        __builtin_amdgcn_s_waitcnt(kWaitVmLgkm0);
-        asm volatile("s_barrier" ::: "memory");
-#pragma unroll
-        for (int k = 0; k < ST; ++k)
-            if (k < (int)nk) {
-#pragma unroll
-                for (int s = 0; s < KS; ++s) {
-                    read(stage[k], s);
-                    mfmas(s);
+            if constexpr (ST > 3) {
+                dma_slice(s_3);
+                next_slice();
+            }
+            __builtin_amdgcn_s_waitcnt(wait_vmcnt_lgkm0((ST - 1) * DMAS));
+            asm volatile("s_barrier" ::: "memory");
+            read(s_0, 0);
+            // Whole rounds of the ring, then the nk % ST slices left (a further
+            // round would multiply zeros: at N = 1024 on three stages 18 slices'
+            // time for 16, at N = 128 on four stages 4 for 2).
+            uint32_t kt = 0;
+            for (; kt + ST <= nk; kt += ST) {
+                step(s_0, s_1);
+                if constexpr (ST == 2) {
+                    step(s_1, s_0);
+                } else if constexpr (ST == 3) {
+                    step(s_1, s_2);
+                    step(s_2, s_0);
+                } else {
+                    step(s_1, s_2);
+                    step(s_2, s_3);
+                    step(s_3, s_0);
                 }
             }
-    } else {
-        dma_slice(s_0);
-        next_slice();
-        dma_slice(s_1);
-        next_slice();
-        if constexpr (ST > 2) {
-            dma_slice(s_2);
-            next_slice();
+            if (kt < nk) step(s_0, s_1);
+            if (ST > 2 && kt + 1 < nk) step(s_1, s_2);
+            if (ST > 3 && kt + 2 < nk) step(s_2, s_3);
         }
-        if constexpr (ST > 3) {
-            dma_slice(s_3);
-            next_slice();
-        }
-        __builtin_amdgcn_s_waitcnt(wait_vmcnt_lgkm0((ST - 1) * DMAS));
-        asm volatile("s_barrier" ::: "memory");
-        read(s_0, 0);
-        // Whole rounds of the ring, then the nk % ST slices left (a further round
-        // would multiply zeros: at N = 1024 on three stages 18 slices' time for 16,
-        // at N = 128 on four stages 4 for 2).
-        uint32_t kt = 0;
-        for (; kt + ST <= nk; kt += ST) {
-            step(s_0, s_1);
-            if constexpr (ST == 2) {
-                step(s_1, s_0);
-            } else if constexpr (ST == 3) {
-                step(s_1, s_2);
-                step(s_2, s_0);
-            } else {
-                step(s_1, s_2);
-                step(s_2, s_3);
-                step(s_3, s_0);
-            }
-        }
-        if (kt < nk) step(s_0, s_1);
-        if (ST > 2 && kt + 1 < nk) step(s_1, s_2);
-        if (ST > 3 && kt + 2 < nk) step(s_2, s_3);
-    }
+    };
+    if (FORM == kGmMixed && split)
+        products(std::bool_constant<FORM == kGmMixed>{});
+    else
+        products(std::bool_constant<false>{});
     // The ring is free for the epilogue once every wave's last reads and
     // (empty) DMA are done.
     __builtin_amdgcn_s_waitcnt(kWaitVmLgkm0);
@@ -601,7 +662,8 @@ __global__ __launch_bounds__(C::THREADS, C::MINB) void gemm_kernel(GemmArgs g) {
     // 32 (JN wc + j) + 8 (v / 4) + 4 (l / 32) + v % 4 (SW: gate v = 8 q + u and
     // up 8 q + 4 + u of column 16 (JN wc + j) + 8 q + 4 (l / 32) + u) of token
     // row 32 (IM wr + i) + l % 32, so v / 4 picks four consecutive outputs of
-    // one token.  Each wave stages its bf16 results (rows of OUTC outputs) in
+    // one token (split: column 32 (JN wc + j) + 16 (v / 8) + 4 (l / 16) + v % 4,
+    // row 32 (IM wr + i) + 16 (v / 4 % 2) + l % 16).  Each wave stages its bf16 results (rows of OUTC outputs) in
     // its part of the first stage, R token blocks at a time, and writes whole
     // 16-byte chunks of token rows.
     constexpr int OUTC = SW ? 16 * JN : 32 * JN;  // a wave's output columns
@@ -637,7 +699,7 @@ __global__ __launch_bounds__(C::THREADS, C::MINB) void gemm_kernel(GemmArgs g) {
 #pragma unroll
         for (int ii = 0; ii < R; ++ii) {
             if (ii >= nb) break;
-            const int i = r0 + ii, t = 32 * ii + (lane & 31);
+            const int i = r0 + ii;
 #pragma unroll
             for (int j = 0; j < JN; ++j)
 #pragma unroll
@@ -651,9 +713,13 @@ __global__ __launch_bounds__(C::THREADS, C::MINB) void gemm_kernel(GemmArgs g) {
                         else
                             e[u] = acc[i][j][4 * q + u];
                     }
-                    const int pc = ep_chunk<CR>((SW ? 2 : 4) * j + q, t);
-                    const int h = (lane >> 5) ^ ep_swap<CR>(t);
-                    ep_write(area + t * OUTC + 8 * pc + 4 * h, pack_bf16x2(e[0], e[1]),
+                    int t = 32 * ii + lane % 32, c = (SW ? 2 : 4) * j + q, h = lane / 32;
+                    if (FORM == kGmMixed && split) {
+                        t = 32 * ii + 16 * (q % 2) + lane % 16;
+                        c = 4 * j + 2 * (q / 2) + lane / 32;
+                        h = lane / 16 % 2;
+                    }
+                    ep_write(area + t * OUTC + 8 * ep_chunk<CR>(c, t) + 4 * (h ^ ep_swap<CR>(t)), pack_bf16x2(e[0], e[1]),
                              pack_bf16x2(e[2], e[3]));
                 }
         }
@@ -706,12 +772,21 @@ uint32_t gemm_tiles(const GemmArgs& g) {
 
 template <typename C, bool SW = false>
 hipError_t gemm_launch(const GemmArgs& g, hipStream_t stream) {
+    const uint32_t tiles = gemm_tiles<C, SW>(g);
     if (g.N / kGmBK <= C::ST)
-        gemm_kernel<C, SW, true><<<gemm_tiles<C, SW>(g), C::THREADS, 0, stream>>>(g);
+        gemm_kernel<C, SW, kGmShort><<<tiles, C::THREADS, 0, stream>>>(g);
     else
-        gemm_kernel<C, SW, false><<<gemm_tiles<C, SW>(g), C::THREADS, 0, stream>>>(g);
+        gemm_kernel<C, SW, kGmRing><<<tiles, C::THREADS, 0, stream>>>(g);
     return hipGetLastError();
 }
+
+template <typename C>
+hipError_t gemm_launch_mixed(const GemmArgs& g, hipStream_t stream) {
+    gemm_kernel<C, false, kGmMixed><<<gemm_tiles<C>(g), C::THREADS, 0, stream>>>(g);
+    return hipGetLastError();
+}
+
+}  // namespace
 
 int gemm_cus() {
     static int cus = [] {
@@ -724,6 +799,8 @@ int gemm_cus() {
     return cus;
 }
 
+namespace {
+
 template <typename C, bool SW>
 float gemm_cost(const GemmArgs& g, uint32_t cus) {
     const float tiles = (float)gemm_tiles<C, SW>(g);
@@ -735,28 +812,45 @@ float gemm_cost(const GemmArgs& g, uint32_t cus) {
 // The configuration of least modelled cost, or the one that the caller names.
 // Every one sums K in the same MFMA order, so the choice does not change a
 // result bit.
-template <bool SW>
-hipError_t gemm_pick_launch(const GemmArgs& g, hipStream_t stream) {
+struct GmPick {
+    const GemmArgs& g;
     const uint32_t cus = (uint32_t)gemm_cus();
     hipError_t (*best)(const GemmArgs&, hipStream_t) = nullptr;
     float least = 0.0f;
     int tile = 0;
-    auto consider = [&](float cost, hipError_t (*launch)(const GemmArgs&, hipStream_t)) {
+    template <typename C, bool SW>
+    void consider(hipError_t (*launch)(const GemmArgs&, hipStream_t)) {
+        const float cost = gemm_cost<C, SW>(g, cus);
         if (g.tile ? ++tile == g.tile : best == nullptr || cost < least) {
             least = cost;
             best = launch;
         }
-    };
-    consider(gemm_cost<GmMini, SW>(g, cus), gemm_launch<GmMini, SW>);
-    consider(gemm_cost<GmSix, SW>(g, cus), gemm_launch<GmSix, SW>);
-    consider(gemm_cost<GmFlat, SW>(g, cus), gemm_launch<GmFlat, SW>);
-    consider(gemm_cost<GmDeep, SW>(g, cus), gemm_launch<GmDeep, SW>);
-    consider(gemm_cost<GmTall, SW>(g, cus), gemm_launch<GmTall, SW>);
-    consider(gemm_cost<GmHalf, SW>(g, cus), gemm_launch<GmHalf, SW>);
-    consider(gemm_cost<GmWide, SW>(g, cus), gemm_launch<GmWide, SW>);
-    consider(gemm_cost<GmBroad, SW>(g, cus), gemm_launch<GmBroad, SW>);
-    consider(gemm_cost<GmLarge, SW>(g, cus), gemm_launch<GmLarge, SW>);
-    return best(g, stream);
+    }
+};
+
+template <bool SW>
+hipError_t gemm_pick_launch(const GemmArgs& g, hipStream_t stream) {
+    GmPick p{g};
+    p.consider<GmMini, SW>(gemm_launch<GmMini, SW>);
+    p.consider<GmSix, SW>(gemm_launch<GmSix, SW>);
+    p.consider<GmFlat, SW>(gemm_launch<GmFlat, SW>);
+    p.consider<GmDeep, SW>(gemm_launch<GmDeep, SW>);
+    p.consider<GmTall, SW>(gemm_launch<GmTall, SW>);
+    p.consider<GmHalf, SW>(gemm_launch<GmHalf, SW>);
+    p.consider<GmWide, SW>(gemm_launch<GmWide, SW>);
+    p.consider<GmBroad, SW>(gemm_launch<GmBroad, SW>);
+    p.consider<GmLarge, SW>(gemm_launch<GmLarge, SW>);
+    return p.best(g, stream);
+}
+
+// The tiles that few tokens leave in question.
+hipError_t gemm_pick_launch_mixed(const GemmArgs& g, hipStream_t stream) {
+    GmPick p{g};
+    p.consider<GmMini, false>(gemm_launch_mixed<GmMini>);
+    p.consider<GmSix, false>(gemm_launch_mixed<GmSix>);
+    p.consider<GmFlat, false>(gemm_launch_mixed<GmFlat>);
+    p.consider<GmDeep, false>(gemm_launch_mixed<GmDeep>);
+    return p.best(g, stream);
 }
 
 }  // namespace
@@ -790,24 +884,20 @@ hipError_t launch_batch_proj_bf16(const uint16_t* W, const uint16_t* x, uint16_t
 }
 
 hipError_t launch_gemm(const GemmArgs& g, hipStream_t stream) {
-    if (g.tile)
-        return g.swiglu ? gemm_pick_launch<true>(g, stream) : gemm_pick_launch<false>(g, stream);
-    if (g.swiglu)
-        return proj_uses_skinny(g.T, g.rows[0]) ? launch_gemm_skinny(g, stream)
-                                                : gemm_pick_launch<true>(g, stream);
-    // The segments of each kind in one launch.
-    GemmArgs part[2] = {g, g};
-    part[0].nseg = part[1].nseg = 0;
+    int split = 0;  // segments summed in the few-token kernel's order
+    uint64_t blocks = 0;
     for (int s = 0; s < g.nseg; ++s) {
-        GemmArgs& p = part[proj_uses_skinny(g.T, g.rows[s])];
-        p.w[p.nseg] = g.w[s];
-        p.y[p.nseg] = g.y[s];
-        p.rows[p.nseg++] = g.rows[s];
+        split += proj_uses_skinny(g.T, g.rows[s], g.N);
+        blocks += skinny_tiles(g.T, g.rows[s]);
     }
-    hipError_t e = hipSuccess;
-    if (part[0].nseg) e = gemm_pick_launch<false>(part[0], stream);
-    if (e == hipSuccess && part[1].nseg) e = launch_gemm_skinny(part[1], stream);
-    return e;
+    if (g.swiglu)
+        return split && !g.tile ? launch_gemm_skinny(g, stream) : gemm_pick_launch<true>(g, stream);
+    if (split == 0) return gemm_pick_launch<false>(g, stream);
+    // A segment alone, or a stack that is one round of the few-token kernel's
+    // blocks as well.
+    if (!g.tile && (g.nseg == 1 || (split == g.nseg && blocks <= kSkinnyRound)))
+        return launch_gemm_skinny(g, stream);
+    return gemm_pick_launch_mixed(g, stream);
 }
 
 }  // namespace tiattn

@@ -30,7 +30,7 @@ constexpr int kSkThreads = 64 * kSkWaves;
 constexpr int kSkChunk = 64;  // K columns per chunk: one 128-byte line of each row
 
 // A wave's LDS slot holds one chunk of its JN + IM 16-row blocks; DEPTH slots
-// per wave, as many as 160 KB hold, are in flight at a time.
+// per wave, at most four and as many as 160 KB hold, are in flight at a time.
 constexpr int sk_depth(int jn, int im) { return jn + im <= 2 ? 4 : (jn + im <= 3 ? 3 : 2); }
 
 // 128-byte rows, 16-byte chunk q of row r at q ^ sk_swz(r): the 16 consecutive
@@ -245,9 +245,10 @@ template <bool SW>
 hipError_t skinny_pick(const GemmArgs& g, hipStream_t stream) {
     hipError_t (*best)(const GemmArgs&, hipStream_t) = nullptr;
     float least = 0.0f;
+    const float cus = (float)gemm_cus();
     auto consider = [&](uint32_t blocks, float fixed, float round, float k, float load,
                         hipError_t (*launch)(const GemmArgs&, hipStream_t)) {
-        const float rounds = ceilf(blocks / 256.0f), use = blocks / (256.0f * rounds);
+        const float rounds = ceilf(blocks / cus), use = blocks / (cus * rounds);
         const float cost = fixed + rounds * (round + g.N / 1024.0f * (k + load * use));
         if (best == nullptr || cost < least) {
             least = cost;
