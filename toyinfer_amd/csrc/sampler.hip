@@ -233,10 +233,23 @@ __device__ __forceinline__ uint32_t top_mask(const uint32_t (&key)[kSpPer], cons
     return take;
 }
 
+// Bits FROM .. TO of the k-th largest of the 256 values v holds per wave, below
+// the higher bits t (each wave finds them by itself, bit by bit).
+template <int FROM, int TO>
+__device__ __forceinline__ uint32_t kth_bits(uint4 v, uint32_t k, uint32_t t) {
+#pragma unroll
+    for (int bit = FROM; bit >= TO; --bit) {
+        const uint32_t c = t | 1u << bit;
+        const uint32_t n = __popcll(__ballot(v.x >= c)) + __popcll(__ballot(v.y >= c)) +
+                           __popcll(__ballot(v.z >= c)) + __popcll(__ballot(v.w >= c));
+        if (n >= k) t = c;
+    }
+    return t;
+}
+
 // A lower bound of the k-th largest valid key of the workgroup: the k-th
-// largest of the threads' maxima, its upper 16 bits (each wave finds them by
-// itself, bit by bit, from all 256 maxima).  0 when fewer than k threads hold
-// a key.
+// largest of the threads' maxima (left in s_max), its upper 16 bits.  0 when
+// fewer than k threads hold a key.
 __device__ __forceinline__ uint32_t bound_kth(const uint32_t (&key)[kSpPer], uint32_t valid, uint32_t k,
                                               uint32_t* s_max, int slots) {
     uint32_t mx = 0;
@@ -247,25 +260,14 @@ __device__ __forceinline__ uint32_t bound_kth(const uint32_t (&key)[kSpPer], uin
     }
     s_max[threadIdx.x] = mx;
     __syncthreads();
-    const uint4 v = reinterpret_cast<const uint4*>(s_max)[threadIdx.x & 63];
-    uint32_t t = 0;
-#pragma unroll
-    for (int bit = 31; bit >= 16; --bit) {
-        const uint32_t c = t | 1u << bit;
-        const uint32_t n = __popcll(__ballot(v.x >= c)) + __popcll(__ballot(v.y >= c)) +
-                           __popcll(__ballot(v.z >= c)) + __popcll(__ballot(v.w >= c));
-        if (n >= k) t = c;
-    }
-    return t;
+    return kth_bits<31, 16>(reinterpret_cast<const uint4*>(s_max)[threadIdx.x & 63], k, 0);
 }
 
 // Emits the valid keys from that bound on, at least the top k with all ties,
 // if there are at most `room` of them; returns how many there are.
 template <typename F>
-__device__ __forceinline__ uint32_t filter_top(const uint32_t (&key)[kSpPer], uint32_t valid, uint32_t k,
-                                               uint32_t room, uint32_t* s_max, uint32_t* s_cnt,
-                                               int slots, F&& emit) {
-    const uint32_t bound = bound_kth(key, valid, k, s_max, slots);
+__device__ __forceinline__ uint32_t filter_top(const uint32_t (&key)[kSpPer], uint32_t valid, uint32_t room,
+                                               uint32_t bound, uint32_t* s_cnt, int slots, F&& emit) {
     uint32_t take = 0;
 #pragma unroll
     for (int j = 0; j < kSpPer; ++j) {
@@ -287,6 +289,45 @@ __device__ __forceinline__ uint32_t filter_top(const uint32_t (&key)[kSpPer], ui
     return total;
 }
 
+// The k-th largest key after a filter that let through too many, without the
+// select's four passes where it is among many equals (rows of equal or masked
+// keys) or, in a chunk, almost always.
+// CHUNK: all bits of the k-th largest of the maxima, if fewer than k keys lie
+// above it (then k keys lie at or above it).  Candidates, of which a thread
+// holds neighbours, so that one chunk's top keys share few threads: any key with
+// the bound's upper 16 bits, if the top k end among its equals.
+// V = 151936, k = 20: all equal 38.5 us by the select alone, 40.4 after the filter,
+// 28.3 so; 300 tokens allowed 31.5, 30.0, 22.5.  need 0: not found.
+template <bool CHUNK>
+__device__ __forceinline__ Sel kth_after_filter(const uint32_t (&key)[kSpPer], uint32_t valid, uint32_t k,
+                                                uint32_t bound, const uint32_t* s_max, uint32_t* s_cnt,
+                                                int slots) {
+    uint32_t t;
+    if constexpr (CHUNK) {
+        t = kth_bits<15, 0>(reinterpret_cast<const uint4*>(s_max)[threadIdx.x & 63], k, bound);
+    } else {
+#pragma unroll
+        for (int j = 0; j < kSpPer; ++j) {
+            if (j >= slots) break;
+            // (whichever lane's write lands last)
+            if ((valid >> j & 1u) && key[j] >> 16 == bound >> 16) s_cnt[1] = key[j];
+        }
+        __syncthreads();
+        t = s_cnt[1];
+    }
+    uint32_t n = 0;  // keys above t, and equal ones in the upper half (8192 at most)
+#pragma unroll
+    for (int j = 0; j < kSpPer; ++j) {
+        if (j >= slots) break;
+        if (valid >> j & 1u) n += key[j] > t ? 1u : (key[j] == t ? 0x10000u : 0u);
+    }
+    const uint32_t sum = wave_scan_incl(n);
+    if ((threadIdx.x & 63) == 63) atomicAdd(s_cnt, sum);
+    __syncthreads();
+    const uint32_t above = *s_cnt & 0xffffu, eq = *s_cnt >> 16;
+    return {t, above < k && above + eq >= k ? k - above : 0u, eq};
+}
+
 // Slots 0..k-1 for the set bits of `take` across the workgroup (any order):
 // a wave scan of the per-thread counts and one LDS atomic per wave.
 template <typename F>
@@ -301,6 +342,28 @@ __device__ __forceinline__ void emit_top(uint32_t take, uint32_t k, int slots, u
 #pragma unroll
     for (int j = 0; j < kSpPer; ++j)
         if (j < slots && (take >> j & 1u) && slot < k) emit(slot++, j);  // exactly k bits are set
+}
+
+// Emits the top k of the workgroup's valid keys, all of them and up to `room`
+// keys by the filter, or exactly k; returns how many.  s_cnt: four words, 0.
+// Candidates of which the filter passes fewer than half are not equals: select.
+template <bool CHUNK, typename F>
+__device__ __forceinline__ uint32_t emit_selected(const uint32_t (&key)[kSpPer], const uint32_t (&idx)[kSpPer],
+                                                  uint32_t valid, uint32_t k, bool filter, uint32_t room,
+                                                  uint32_t* s_max, uint32_t* s_cnt, uint32_t* s_hist,
+                                                  int slots, F&& emit) {
+    uint32_t n = ~0u, bound = 0;
+    if (filter) {
+        bound = bound_kth(key, valid, k, s_max, slots);
+        n = filter_top(key, valid, room, bound, s_cnt, slots, emit);
+        if (n <= room) return n;
+    }
+    Sel s = {0, 0, 0};
+    if (filter && (CHUNK || n >= kSpBlocksSmallK * k / 2))
+        s = kth_after_filter<CHUNK>(key, valid, k, bound, s_max, s_cnt + 1, slots);
+    if (s.need == 0) s = select_kth(key, valid, k, s_hist, slots);
+    emit_top(top_mask(key, idx, valid, s, s_hist, slots), k, slots, s_cnt + 3, emit);
+    return k;
 }
 
 // SplitMix64 finaliser (Steele, Lea and Flood, "Fast splittable pseudorandom
@@ -328,14 +391,12 @@ __device__ __forceinline__ void sp_write(const SampleArgs& a, uint32_t p_out, ui
 
 __global__ __launch_bounds__(kSpThreads) void sample_kernel(SampleArgs a) {
     __shared__ __align__(16) uint32_t s_hist[2 * kSpWaves * 256];
-    __shared__ uint32_t s_wu[kSpWaves];
     __shared__ float s_wf[kSpWaves];
     __shared__ __align__(16) uint32_t s_max[kSpThreads];
     __shared__ uint64_t s_top[kSampleMaxK];
     __shared__ uint64_t s_sorted[64];
     __shared__ float s_acc[kSampleMaxK];
-    // Emitted keys: by the filter and by the select, of either phase.
-    __shared__ uint32_t s_res[2], s_cnt[4];
+    __shared__ uint32_t s_res[2], s_cnt[8];  // s_cnt: emit_selected's, of either phase
     __shared__ bool s_last;
 
     const uint32_t k = a.k, tid = threadIdx.x;
@@ -346,7 +407,7 @@ __global__ __launch_bounds__(kSpThreads) void sample_kernel(SampleArgs a) {
     const uint32_t width = sp_width(a.n, k);
     const bool filter = width != k;
     uint32_t* ws_idx = ws_key + G * width;
-    if (tid < 4) s_cnt[tid] = 0;
+    if (tid < 8) s_cnt[tid] = 0;
 
     // Phase 1: this workgroup's chunk, element j*256 + t in thread t's key[j].
     const uint32_t cs = (a.n + G - 1) / G;
@@ -388,13 +449,8 @@ __global__ __launch_bounds__(kSpThreads) void sample_kernel(SampleArgs a) {
             bk[slot] = key[j];
             bi[slot] = idx[j];
         };
-        uint32_t n = filter ? filter_top(key, valid, k, width, s_max, &s_cnt[0], slots, emit) : ~0u;
-        if (n > width) {
-            const Sel s = select_kth(key, valid, k, s_hist, slots);
-            const uint32_t take = top_mask(key, idx, valid, s, s_hist, slots);
-            emit_top(take, k, slots, &s_cnt[1], emit);
-            n = k;
-        }
+        const uint32_t n =
+            emit_selected<true>(key, idx, valid, k, filter, width, s_max, s_cnt, s_hist, slots, emit);
         if (tid >= n && tid < width) {
             bk[tid] = 0u;
             bi[tid] = 0xffffffffu;
@@ -439,13 +495,7 @@ __global__ __launch_bounds__(kSpThreads) void sample_kernel(SampleArgs a) {
         auto emit = [&](uint32_t slot, int j) {
             s_top[slot] = ((uint64_t)key[j] << 32) | (uint32_t)~idx[j];
         };
-        found = filter ? filter_top(key, valid, k, 64, s_max, &s_cnt[2], slots, emit) : ~0u;
-        if (found > 64) {
-            const Sel s = select_kth(key, valid, k, s_hist, slots);
-            const uint32_t take = top_mask(key, idx, valid, s, s_hist, slots);
-            emit_top(take, k, slots, &s_cnt[3], emit);
-            found = k;
-        }
+        found = emit_selected<false>(key, idx, valid, k, filter, 64, s_max, s_cnt + 4, s_hist, slots, emit);
     }
     uint32_t p_out = 0;
     if (a.pos) p_out = *a.pos;
