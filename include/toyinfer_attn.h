@@ -66,10 +66,15 @@ int toyinfer_flash_attention_algo_bf16(const void* Qs, const void* Ks, const voi
  * batch_rope_bf16 on Q and K followed by flash_attention_v1_bf16, as
  * src/transformer.cpp:380-404 sequences them.  The rotation angles come from
  * rope_cos_sin [>= S][D/2][2] (fp32 (cos, sin), 16-byte aligned), built once
- * per model with toyinfer_rope_cos_sin_f32.  Q_raw is read only (normalised
- * and rotated on load); the normalised and rotated K is written to K_out
- * [S][Hkv][D] (may alias K_raw; typically the layer's KV-cache slot), then
- * used as the attention's K.  All tensor pointers 16-byte aligned. */
+ * per model with toyinfer_rope_cos_sin_f32.  The normalised and rotated K is
+ * written to K_out [S][Hkv][D] (may alias K_raw; typically the layer's KV-cache
+ * slot), then used as the attention's K.  Q_raw is not written, unless it is Os:
+ * Os may be Q_raw, or overlap K_raw where K_out does not.  At the lengths that
+ * toyinfer_flash_attention_v1_bf16 runs split over the keys, Os holds the
+ * normalised and rotated Q before it holds the output; above them Q is
+ * transformed as it is loaded.  Os over Vs or K_out works only while no other
+ * query row or head reads what a row's output overwrites (S <= 32 and Hq ==
+ * Hkv).  All tensor pointers 16-byte aligned. */
 int toyinfer_prefill_qknorm_rope_attention_bf16(
     const void* Q_raw, const void* K_raw, const void* Vs, void* Os, void* K_out,
     const void* q_gamma, const void* k_gamma, const float* rope_cos_sin, float rms_norm_eps,

@@ -208,6 +208,33 @@ def test_fused_prefill_prepared_q(dev, s, hq, hkv, d, o_is):
     assert np.array_equal(H.from_dev_bf16(o), H.from_dev_bf16(exp))
 
 
+@pytest.mark.parametrize("s,h,d", [(1, 2, 64), (31, 8, 128), (32, 4, 64)])
+@pytest.mark.parametrize("over", ["v", "k_out", "q_next"])
+def test_fused_prefill_output_over_an_input(dev, s, h, d, over):
+    """One query tile and as many query as KV heads: each workgroup reads its
+    head's rows before it writes the same columns, so the output may lie over V,
+    over K_out, or over Q one token further on."""
+    print(f"[fused] output over {over} S={s} {h}/{h} D={d}", flush=True)
+    qb, kb, vb, gq, gk = config4_inputs(s, h, h, d, seed=8)
+    exp, k_exp, _ = fused_prefill(qb, kb, vb, gq, gk, 1e-6, 1e6, dev)
+    k, v = H.to_dev_bf16(kb, dev), H.to_dev_bf16(vb, dev)
+    buf = torch.zeros((s + 1, h, d), dtype=torch.bfloat16, device=dev)
+    buf[:s] = H.to_dev_bf16(qb, dev)
+    k_out = torch.empty_like(k)
+    o = {"v": v, "k_out": k_out, "q_next": buf[1:]}[over]
+    f = torch.empty(d // 2, dtype=torch.float32, device=dev)
+    attn.precompute_freq_f32(f, d, 1e6)
+    table = torch.empty((s, d // 2, 2), dtype=torch.float32, device=dev)
+    attn.rope_cos_sin_f32(table, f, s, d)
+    attn.prefill_qknorm_rope_attention_bf16(buf[:s], k, v, o, k_out, H.to_dev_bf16(gq, dev),
+                                            H.to_dev_bf16(gk, dev), table, 1e-6, h, h, d, s)
+    H.sync()
+    if over != "k_out":
+        assert np.array_equal(H.from_dev_bf16(k_out), k_exp)
+    H.check_bar(H.bf16_bits_to_f32(H.from_dev_bf16(o)), H.bf16_bits_to_f32(exp), "output",
+                max_abs=1e-2, mean_abs=2e-4)
+
+
 def test_fused_prefill_head_pairs_ragged_rows(dev):
     """The fused entry at a length where the head-pair 128-row kernel is
     chosen (S = 4100, 32/8: 33 query tiles x 16 pairs, two rounds of the

@@ -193,7 +193,14 @@ int toyinfer_prefill_qknorm_rope_attention_bf16(
     p.hq = num_q_heads;
     p.hkv = num_kv_heads;
     p.d = heads_dim;
-    if (prefill_uses_split(p)) {
+    const size_t row = (size_t)seq_len * heads_dim * 2;
+    // Os holds the prepared Q only where that overwrites nothing still to be
+    // read: an output buffer over V, the attention's K or rows of Q other than
+    // its own keeps Q in registers until the output is written.
+    const bool os_free = !overlap(Os, row * num_q_heads, Vs, row * num_kv_heads) &&
+                         !overlap(Os, row * num_q_heads, K_out, row * num_kv_heads) &&
+                         (Os == Q_raw || !overlap(Os, row * num_q_heads, Q_raw, row * num_q_heads));
+    if (prefill_uses_split(p) && os_free) {
         // Q and K normalised and rotated in one launch, Q into Os: a
         // workgroup of the split kernels reads the Q rows of an item before
         // it writes that item's output, the same rows, and no other
@@ -207,7 +214,6 @@ int toyinfer_prefill_qknorm_rope_attention_bf16(
         const uint16_t* kg = static_cast<const uint16_t*>(k_gamma);
         uint16_t* k_out = static_cast<uint16_t*>(K_out);
         hipError_t e;
-        const size_t row = (size_t)seq_len * heads_dim * 2;
         if (overlap(Os, row * num_q_heads, K_raw, row * num_kv_heads)) {
             // A caller's output buffer may be the K projection's, which is
             // done with once K_out is written: K first, then Q into Os.
