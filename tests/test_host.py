@@ -361,3 +361,18 @@ def test_dropin_header_rejects_illegal_instantiations(tmp_path, bad):
             "void f_(const bf16* q, bf16* o, float* f) { " + bad + " }\n")
     res = compile_snippet(tmp_path, text)
     assert res.returncode != 0 and "static assertion failed" in res.stderr
+
+
+def test_current_stream_without_torchs_raw_lookup(monkeypatch):
+    """A torch without the lookup underneath current_stream(): its public call."""
+    import types
+
+    import torch
+    monkeypatch.setattr(torch.cuda, "is_initialized", lambda: True)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda: types.SimpleNamespace(cuda_stream=42))
+    monkeypatch.delattr(torch._C, "_cuda_getCurrentRawStream", raising=False)
+    attn._current_stream_lookup.cache_clear()
+    try:
+        assert attn._stream(None) == 42
+    finally:
+        attn._current_stream_lookup.cache_clear()

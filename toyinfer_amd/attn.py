@@ -13,6 +13,7 @@ src/kernel_common.cuh:11-20; the C++ drop-in header keeps that behaviour).
 from __future__ import annotations
 
 import ctypes
+import functools
 import os
 from typing import Optional
 
@@ -125,21 +126,32 @@ def _ptr(t) -> Optional[int]:
     return int(t.data_ptr())
 
 
+@functools.lru_cache(maxsize=None)
+def _current_stream_lookup():
+    """torch.cuda.current_stream() builds a Stream object on every call, 3.2 us
+    of a one-kernel call's 7.4 us on the host (3.7 us of it HIP's launch); the
+    same handle comes in 0.2 us from the lookup underneath, where this torch
+    has it."""
+    import torch
+
+    raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+    device = getattr(torch._C, "_cuda_getDevice", None)
+    if raw is None or device is None:
+        return lambda: int(torch.cuda.current_stream().cuda_stream)
+    return lambda: raw(device())
+
+
 def _stream(stream) -> Optional[int]:
     """hipStream_t handle: an int, a torch.cuda.Stream, or None for torch's
-    current stream on the current device.
-
-    torch.cuda.current_stream() builds a Stream object on every call, 3.2 us
-    of a one-kernel call's 7.4 us on the host (3.7 us of it HIP's launch); the
-    same handle comes in 0.2 us from the lookup underneath, once torch has
-    initialised the device (before that, its own error or initialisation)."""
+    current stream on the current device (before torch has initialised the
+    device, by its own call: its error or its initialisation)."""
     if isinstance(stream, int):
         return stream
     import torch
 
     if stream is None:
         if torch.cuda.is_initialized():
-            return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+            return _current_stream_lookup()()
         stream = torch.cuda.current_stream()
     return int(stream.cuda_stream)
 
