@@ -392,8 +392,7 @@ int toyinfer_qwen3_prefill(toyinfer_qwen3* m, const uint32_t* token_ids_d, uint3
         }
         if (split_attn) {
             // Q normalised and rotated in place, K into the cache rows, one
-            // launch; then the split kernel on the prepared Q (its fused-Q
-            // form cannot keep the next item's Q in flight).
+            // launch; then the split kernel on the prepared Q.
             TRYH(launch_qk_norm_rope_rows(m->p_q, m->p_q, u16(L.q_norm), m->p_k, kc,
                                           u16(L.k_norm), m->rope, eps, T, hq, hkv, d, st));
             PrefillProblem pp = attn;
