@@ -261,10 +261,10 @@ def test_gemm_residual_epilogue_equals_projection_then_add(dev, T, H, M):
                                      (17, 256, 200), (33, 256, 204)])
 def test_gemm_swiglu_equals_projections_then_swiglu(dev, T, hid, M):
     """Gate/up with SwiGLU in the epilogue equals the two projections followed
-    by batch_swiglu_bf16x2, bit for bit: the GEMM at sizes of the models, and
-    the few-token kernel (M = 200: a ragged last tile; M = 204: rows not
-    16-byte aligned).  Every GEMM tile size and its ragged tiles:
-    test_gemm_tile_sizes_and_epilogues."""
+    by batch_swiglu_bf16x2, bit for bit, at sizes of the models and at small
+    ones (M = 200: a ragged last tile; M = 204: rows not 16-byte aligned).  Every
+    GEMM tile size and its ragged tiles: test_gemm_tile_sizes_and_epilogues;
+    the few-token kernel: test_few_token_segments_and_epilogues."""
     print(f"[step] gemm swiglu T={T} hid={hid} M={M}", flush=True)
     g = torch.Generator(device=dev).manual_seed(39)
     x = torch.randn((T, hid), generator=g, device=dev).to(torch.bfloat16)
@@ -284,12 +284,15 @@ def test_gemm_swiglu_equals_projections_then_swiglu(dev, T, hid, M):
 
 # The K-split kernel of few tokens: token tiles of 16, 32 and 48 with
 # remainders, output tiles of 16 and 32 with remainders, fewer chunks than
-# waves, uneven shares of K, and both sides of the line to the ring GEMM
-# (T rows <= 327680, T <= 320).
+# waves (N = 320 to 448), uneven shares of K, and both sides of the lines to the
+# GEMM (T rows <= 327680, T <= 320, N > 256, 256 blocks of 32 x 48 below N =
+# 4096; 33 x 8193, 49 x 4097 and 9 x 12289 are more).
 @pytest.mark.parametrize("T,M,N", [(5, 1, 64), (5, 17, 576), (16, 15, 512), (17, 130, 3072),
                                    (48, 1024, 2048), (49, 33, 4160), (80, 4096, 1024),
                                    (81, 4096, 1024), (320, 1024, 1024), (321, 1000, 1024),
-                                   (9, 12289, 128), (37, 8853, 192)])
+                                   (9, 12289, 128), (37, 8853, 192), (5, 17, 320),
+                                   (48, 1000, 448), (33, 8192, 384), (33, 8193, 384),
+                                   (49, 4097, 512), (9, 12289, 4160), (33, 8192, 4096)])
 def test_batch_proj_few_tokens(dev, T, M, N):
     print(f"[step] few tokens T={T} M={M} N={N}", flush=True)
     g = torch.Generator(device=dev).manual_seed(40)
